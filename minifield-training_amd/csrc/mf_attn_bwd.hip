@@ -16,11 +16,12 @@
 //              Q^T read transposed from the Q / dO tiles.  The group's heads
 //              are summed in registers, which is the transpose of the
 //              reference's jnp.repeat of K/V (kernels/attention.py:19-22).
-// The fp32 kernels (parity tests, smoke) stage through registers and read
-// single floats with v_mfma_f32_32x32x2_f32.
+// The fp32 kernels split the same work finer (32 rows and one head per
+// workgroup, the other side over its waves) and use v_mfma_f32_32x32x2_f32.
 // Rows with no valid key have lse = +inf, so their P is exactly 0 and they
 // contribute nothing; their dq is written as 0.
 #include "mf_common.h"
+#include "mf_f32.h"
 #include "mf_lds.h"
 
 namespace mf {
@@ -48,13 +49,12 @@ struct BwdArgs {
   int T, S, Hq, Hkv, G, hchunks;
   int nq, nk, tq_pad, tk_pad;
   int causal;
-  int fuse_delta;  // bf16 dq computes D = rowsum(dO * O) itself and writes -D and lse2
+  int fuse_delta;  // dq computes D = rowsum(dO * O) itself and writes -D and lse2
   float scale, scale_log2;
-  FastDiv div_nh, div_hchunks, div_nq, div_hkv, div_nk, div_g;  // Hkv * hchunks, hchunks, nq, Hkv, nk, G
+  FastDiv div_nh, div_hchunks, div_nq, div_hkv, div_nk, div_g, div_hq;  // Hkv * hchunks, hchunks, nq, Hkv, nk, G, Hq
 };
 
 constexpr int kStep = 64;
-constexpr int kRowF = kD + 1;  // fp32 LDS row pitch
 
 // ---------------------------------------------------------------------------
 // 1. delta
@@ -96,381 +96,334 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(BwdArgs a, int B) {
 }
 
 // ---------------------------------------------------------------------------
-// 2. dq (per query tile), fp32
+// 2. dq, fp32: one workgroup per (32-query block, query head), its four waves
+// on every fourth 32-key block of the tile's list, their dQ added through LDS
+// in wave order (the fp32 forward's split, for the same reason: the kernel is
+// bound by the chain of 64-cycle MFMAs a wave has to run, 96 per block).
+// Measured (same box, us per launch, before -> after): 2 x 256 tokens, 4/2
+// heads, segments 1-64: 59.9 + 6.7 -> 13.1; 2 x 1499, 16/8 heads, causal, mean
+// segment 512: 144 + 8.0 -> 38.8 (the second term is the separate D pass).
 // ---------------------------------------------------------------------------
-struct DqLdsF32 {
-  float k[2][kStep * kRowF];
-  float v[2][kStep * kRowF];
-  int kid[2][kStep];
-};
-
-struct StageF32 {
-  u32x4 r[8];
-};
-
-// K and V rows kb .. kb+63 of one KV head (zero past S) into registers.
-__device__ __forceinline__ void dq_load_f32(const BwdArgs& a, int b, int kvh, int kb, StageF32& st) {
-  const int tid = threadIdx.x;
-  const float* ks = reinterpret_cast<const float*>(a.k);
-  const float* vs = reinterpret_cast<const float*>(a.v);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = tid + 256 * i;
-    const int key = kb + (u >> 4), ch = u & 15;
-    const size_t off = (((size_t)b * a.S + key) * a.Hkv + kvh) * kD + ch * 4;
-    st.r[i] = key < a.S ? ld_u32x4(ks + off) : u32x4{0, 0, 0, 0};
-    st.r[4 + i] = key < a.S ? ld_u32x4(vs + off) : u32x4{0, 0, 0, 0};
-  }
-}
-
-__device__ __forceinline__ void dq_store_f32(const BwdArgs& a, int b, int kb, const StageF32& st,
-                                             DqLdsF32& lds, int buf) {
-  const int tid = threadIdx.x;
-  if (tid < kStep) lds.kid[buf][tid] = a.kid[(size_t)b * a.tk_pad + kb + tid];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = tid + 256 * i;
-    const int key = u >> 4, ch = u & 15;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      lds.k[buf][key * kRowF + ch * 4 + e] = __uint_as_float(st.r[i][e]);
-      lds.v[buf][key * kRowF + ch * 4 + e] = __uint_as_float(st.r[4 + i][e]);
-    }
-  }
-}
-
-template <int HPW>
-__global__ __launch_bounds__(256) void bwd_dq_f32_kernel(BwdArgs a) {
-  __shared__ DqLdsF32 lds;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void bwd_dq_f32_kernel(BwdArgs a) {
+  __shared__ F32Tile kt[4], vt[4], qt;  // the waves' K and V blocks; the queries
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int half = lane >> 5;
-  // 1-D grid: (query-tile item in launch order, kvh, head chunk), heads fastest
-  const int nh = a.Hkv * a.hchunks;
-  const int slot = uniform(fast_div(blockIdx.x, a.div_nh));
-  const int hr = uniform(blockIdx.x - slot * nh);
-  const int kvh = uniform(fast_div(hr, a.div_hchunks));
-  const int hc = uniform(hr - kvh * a.hchunks);
-  const int item = ld_const(a.qorder, slot);  // (row, query tile), longest first
-  const int b = uniform(fast_div(item, a.div_nq));
-  const int qt = uniform(item - b * a.nq);
-  const int qpos = qt * kTile + wave * 32 + (lane & 31);
+  const int wave = uniform(threadIdx.x >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  F32Unit w;
+  if (!f32_unit(a.qorder, a.div_hq, a.div_hkv, a.div_nq, a.T, a.G, w)) return;
+  const int b = w.b, q0 = w.row0;
+  const int qpos = q0 + col;
+  const int qrow = min(qpos, a.T - 1);
   const int myqid = a.qid[(size_t)b * a.tq_pad + qpos];
-  const bool qvalid = qpos < a.T;
-  const bool qactive = qvalid && myqid != 0;
-  int head[HPW];
-#pragma unroll
-  for (int j = 0; j < HPW; ++j) head[j] = kvh * a.G + hc * HPW + j;
+  const int u = uniform(myqid);
+  const bool quni = __all(myqid == u);
+  const bool qactive = qpos < a.T && myqid != 0;
 
-  float qf[HPW][32], gf[HPW][32];
-  float lse2[HPW], dlt[HPW];
+  constexpr size_t kRow = kD * sizeof(float);
+  const size_t q_off = ((size_t)b * a.T * a.Hq + w.head) * kRow;
+  const uint32_t q_stride = (uint32_t)(a.Hq * kRow);
+  f32x4 kx[8], vx[8];  // rows in flight
+  f32x4 gf[8];         // the lane's dO operand, through the wave's V tile
+  f32_load(reinterpret_cast<const char*>(a.dout) + q_off, q_stride, q0, a.T - 1, lane, vx);
+  if (wave == 0)
+    f32_load(reinterpret_cast<const char*>(a.q) + q_off, q_stride, q0, a.T - 1, lane, kx);
+  f32_store(vt[wave], lane, vx);
+  if (wave == 0) f32_store(qt, lane, kx);
+  if (a.fuse_delta)
+    f32_load(reinterpret_cast<const char*>(a.out) + q_off, q_stride, q0, a.T - 1, lane, kx);
+  wave_lds_fence();
 #pragma unroll
-  for (int j = 0; j < HPW; ++j) {
-    const size_t row = (((size_t)b * a.T + qpos) * a.Hq + head[j]) * kD;
-    const float* qs = reinterpret_cast<const float*>(a.q) + row + half;
-    const float* gs = reinterpret_cast<const float*>(a.dout) + row + half;
+  for (int j = 0; j < 8; ++j) gf[j] = vt[wave].row4(lane, j);
+  const size_t li = ((size_t)b * a.Hq + w.head) * a.T + qrow;
+  float nd;  // -D
+  if (a.fuse_delta) {
+    f32_store(kt[wave], lane, kx);  // O
+    wave_lds_fence();
+    float part = 0.f;
 #pragma unroll
-    for (int st = 0; st < 32; ++st) {
-      qf[j][st] = qvalid ? qs[2 * st] : 0.f;
-      gf[j][st] = qvalid ? gs[2 * st] : 0.f;
+    for (int j = 0; j < 8; ++j) {
+      const f32x4 ox = kt[wave].row4(lane, j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part = fmaf(ox[e], gf[j][e], part);
     }
-    const size_t li = ((size_t)b * a.Hq + head[j]) * a.T + qpos;
-    lse2[j] = qactive ? a.lse[li] * kLog2e : kPosInf;
-    dlt[j] = qvalid ? -a.ndelta[li] : 0.f;
+    nd = -halves_sum(part);
+  } else {
+    nd = a.ndelta[li];
+  }
+  const float lse2 = qactive ? a.lse[li] * kLog2e : kPosInf;
+  nd = qactive ? nd : 0.f;
+  if (a.fuse_delta && wave == 0 && half == 0 && qpos < a.T) {
+    a.ndelta[li] = nd;
+    a.lse2[li] = lse2;
   }
 
-  f32x16 dqacc[HPW][2];
-#pragma unroll
-  for (int j = 0; j < HPW; ++j) {
-    dqacc[j][0] = zero16();
-    dqacc[j][1] = zero16();
-  }
-
-  const int count = ld_const(a.qcnt, b * a.nq + qt);
-  const int* list = a.qlist + ((size_t)b * a.nq + qt) * 2 * a.nk;
-  const int nsteps = count;  // one 64-key stage per list entry
+  f32x16 dqacc[2] = {zero16(), zero16()};
   const float c = a.scale_log2;
+  const int* list = a.qlist + ((size_t)b * a.nq + w.tile) * 2 * a.nk;
+  const int nb = 2 * ld_const(a.qcnt, b * a.nq + w.tile);  // 32-key blocks
+  const int* kid_row = a.kid + (size_t)b * a.tk_pad;
+  const char* kg = reinterpret_cast<const char*>(a.k) + ((size_t)b * a.S * a.Hkv + w.kvh) * kRow;
+  const char* vg = reinterpret_cast<const char*>(a.v) + ((size_t)b * a.S * a.Hkv + w.kvh) * kRow;
+  const uint32_t kv_stride = (uint32_t)(a.Hkv * kRow);
 
-  StageF32 stage;
-  if (nsteps > 0) {
-    const int kb0 = (list[0] >> 2) * kStep;
-    dq_load_f32(a, b, kvh, kb0, stage);
-    dq_store_f32(a, b, kb0, stage, lds, 0);
-  }
+  int kidl = 0, entry = 0, k0 = 0;
+  // (as in the forward: stages ascend, so a block past the queries ends it)
+  auto fetch = [&](int i) {
+    if (i >= nb) return false;
+    entry = ld_const(list, i >> 1);
+    k0 = (entry >> 2) * kStep + (i & 1) * 32;
+    if (a.causal && k0 > q0 + 31) return false;
+    kidl = kid_row[k0 + col];
+    f32_load(kg, kv_stride, k0, a.S - 1, lane, kx);
+    f32_load(vg, kv_stride, k0, a.S - 1, lane, vx);
+    return true;
+  };
+  int i = wave;
+  bool more = fetch(i);
   __syncthreads();
-
-  for (int step = 0; step < nsteps; ++step) {
-    const int buf = step & 1;
-    const int entry = list[step];
-    const int kb = (entry >> 2) * kStep;
-    const bool partial = (entry & 3) == 1;
-    int next_kb = 0;
-    if (step + 1 < nsteps) {
-      next_kb = (list[step + 1] >> 2) * kStep;
-      dq_load_f32(a, b, kvh, next_kb, stage);
+  while (more) {
+    const int kb = k0;
+    bool run = true, mask_ids = false, diag = false;
+    if ((entry & 3) == 1) {
+      diag = a.causal && kb + 31 > q0;
+      mask_ids = true;
+      if (quni) {
+        const uint64_t same = __ballot(kidl == u);
+        run = u != 0 && same != 0;
+        mask_ids = same != ~0ull;
+      }
     }
-
+    i += 4;
+    if (!run) {
+      more = fetch(i);
+      continue;
+    }
+    wave_lds_fence();
+    f32_store(kt[wave], lane, kx);
+    f32_store(vt[wave], lane, vx);
+    wave_lds_fence();
+    more = fetch(i);
+    f32x16 s = zero16(), dp;
 #pragma unroll
-    for (int kb2 = 0; kb2 < 2; ++kb2) {
-      f32x16 s[HPW], dp[HPW];
+    for (int r = 0; r < 16; ++r) dp[r] = nd;
 #pragma unroll
-      for (int j = 0; j < HPW; ++j) {
-        s[j] = zero16();
-        dp[j] = zero16();
+    for (int j = 0; j < 8; ++j) {
+      const f32x4 kr = kt[wave].row4(lane, j), qr = qt.row4(lane, j);
+      const f32x4 vr = vt[wave].row4(lane, j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s = mfma32x32x2(kr[e], qr[e], s);
+        dp = mfma32x32x2(vr[e], gf[j][e], dp);
       }
-      const float* krow = &lds.k[buf][(kb2 * 32 + (lane & 31)) * kRowF + half];
-      const float* vrow = &lds.v[buf][(kb2 * 32 + (lane & 31)) * kRowF + half];
-#pragma unroll
-      for (int st = 0; st < 32; ++st) {
-        const float kf = krow[2 * st];
-        const float vf = vrow[2 * st];
-#pragma unroll
-        for (int j = 0; j < HPW; ++j) {
-          s[j] = mfma32x32x2(kf, qf[j][st], s[j]);
-          dp[j] = mfma32x32x2(vf, gf[j][st], dp[j]);
-        }
-      }
-      // P^T and dS^T in place of s
+    }
+    if (mask_ids) {
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        bool ok[4] = {true, true, true, true};
-        if (partial) {
-          const int kk0 = kb2 * 32 + 8 * g4 + 4 * half;
-          const int4 kids = *reinterpret_cast<const int4*>(&lds.kid[buf][kk0]);
-          const int kv[4] = {kids.x, kids.y, kids.z, kids.w};
+        const int4 kids = *reinterpret_cast<const int4*>(&kid_row[kb + 8 * g4 + 4 * half]);
+        const int kv[4] = {kids.x, kids.y, kids.z, kids.w};
 #pragma unroll
-          for (int i = 0; i < 4; ++i) ok[i] = kv[i] == myqid && (!a.causal || kb + kk0 + i <= qpos);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = g4 * 4 + i;
-#pragma unroll
-          for (int j = 0; j < HPW; ++j) {
-            const float p = ok[i] ? fast_exp2(fmaf(s[j][r], c, -lse2[j])) : 0.f;
-            s[j][r] = p * (dp[j][r] - dlt[j]);
-          }
-        }
+        for (int e = 0; e < 4; ++e) s[g4 * 4 + e] = kv[e] == myqid ? s[g4 * 4 + e] : kNegInf;
       }
-      // dQ^T += K^T dS^T
-#pragma unroll
-      for (int db = 0; db < 2; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float af = lds.k[buf][(kb2 * 32 + acc_row(r, lane)) * kRowF + db * 32 + (lane & 31)];
-#pragma unroll
-          for (int j = 0; j < HPW; ++j) dqacc[j][db] = mfma32x32x2(af, s[j][r], dqacc[j][db]);
-        }
     }
-
-    if (step + 1 < nsteps) dq_store_f32(a, b, next_kb, stage, lds, buf ^ 1);
-    __syncthreads();
+    if (diag) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = kb + acc_row(r, lane) <= qpos ? s[r] : kNegInf;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(fmaf(s[r], c, -lse2)) * dp[r];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      dqacc[0] = mfma32x32x2(kt[wave].col(lane, 0, r), s[r], dqacc[0]);
+      dqacc[1] = mfma32x32x2(kt[wave].col(lane, 1, r), s[r], dqacc[1]);
+    }
   }
 
-  if (!qvalid) return;
+  wave_lds_fence();
+  f32_put(kt[wave], lane, dqacc);
+  __syncthreads();
+  const int eq = threadIdx.x >> 3, d0 = 8 * (threadIdx.x & 7);
+  if (q0 + eq >= a.T) return;
+  const bool keep = a.qid[(size_t)b * a.tq_pad + q0 + eq] != 0;
+  float* dst = reinterpret_cast<float*>(reinterpret_cast<char*>(a.dq) + q_off +
+                                        (size_t)(q0 + eq) * q_stride) + d0;
 #pragma unroll
-  for (int j = 0; j < HPW; ++j) {
+  for (int h = 0; h < 2; ++h) {
+    f32x4 o = f32_sum(kt, eq, d0 + 4 * h);
 #pragma unroll
-    for (int db = 0; db < 2; ++db)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int d0 = db * 32 + 8 * g4 + 4 * half;
-        const size_t off = (((size_t)b * a.T + qpos) * a.Hq + head[j]) * kD + d0;
-        f32x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = qactive ? dqacc[j][db][g4 * 4 + i] * a.scale : 0.f;
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.dq) + off) = o;
-      }
+    for (int e = 0; e < 4; ++e) o[e] = keep ? o[e] * a.scale : 0.f;
+    *reinterpret_cast<f32x4*>(dst + 4 * h) = o;
   }
 }
 
 // ---------------------------------------------------------------------------
-// 3. dk, dv (per key tile and KV head), fp32
+// 3. dk, dv, fp32: one workgroup per (32-key block, KV head), its eight waves
+// on every eighth (32-query block, head of the group) pair, their dK and dV
+// added through LDS in wave order.  Eight waves, not
+// four: the longest tile's chain of iterations ends the launch.  Measured (as
+// above): 73.6 -> 17.4; 215 -> 46.4 (with the rows read from memory in operand
+// order: 59.4 with eight waves, 71.4 with four).
 // ---------------------------------------------------------------------------
-struct KvLdsF32 {
-  float q[2][kStep * kRowF];
-  float g[2][kStep * kRowF];
-  float lse2[2][kStep];
-  float dlt[2][kStep];
-  int qid[2][kStep];
-};
+constexpr int kKvWaves = 8;
+constexpr int kKvDims = 32 * kD / (64 * kKvWaves);  // outputs per thread
 
-struct KvStageF32 {
-  u32x4 r[8];
-  float lse2, dlt;
-  int qid;
-};
-
-// Iteration `it` of a key tile's loop -> (64-query stage entry, head in group).
-__device__ __forceinline__ void kv_iter(const BwdArgs& a, const int* list, int it, int& qb,
-                                        int& head_in_group, int& cls) {
-  const int entry = list[it / a.G];
-  head_in_group = it % a.G;
-  qb = (entry >> 2) * kStep;
-  cls = entry & 3;
-}
-
-__device__ __forceinline__ void kv_load_f32(const BwdArgs& a, int b, int h, int qb, KvStageF32& st) {
-  const int tid = threadIdx.x;
-  const float* qs = reinterpret_cast<const float*>(a.q);
-  const float* gs = reinterpret_cast<const float*>(a.dout);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = tid + 256 * i;
-    const int qq = qb + (u >> 4), ch = u & 15;
-    const size_t off = (((size_t)b * a.T + qq) * a.Hq + h) * kD + ch * 4;
-    st.r[i] = qq < a.T ? ld_u32x4(qs + off) : u32x4{0, 0, 0, 0};
-    st.r[4 + i] = qq < a.T ? ld_u32x4(gs + off) : u32x4{0, 0, 0, 0};
-  }
-  if (tid < kStep) {
-    const int qq = qb + tid;
-    const int id = a.qid[(size_t)b * a.tq_pad + qq];
-    const bool act = qq < a.T && id != 0;
-    const size_t li = ((size_t)b * a.Hq + h) * a.T + qq;
-    st.qid = id;
-    st.lse2 = act ? a.lse[li] * kLog2e : kPosInf;
-    st.dlt = act ? -a.ndelta[li] : 0.f;
-  }
-}
-
-__device__ __forceinline__ void kv_store_f32(const KvStageF32& st, KvLdsF32& lds, int buf) {
-  const int tid = threadIdx.x;
-  if (tid < kStep) {
-    lds.qid[buf][tid] = st.qid;
-    lds.lse2[buf][tid] = st.lse2;
-    lds.dlt[buf][tid] = st.dlt;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = tid + 256 * i;
-    const int qq = u >> 4, ch = u & 15;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      lds.q[buf][qq * kRowF + ch * 4 + e] = __uint_as_float(st.r[i][e]);
-      lds.g[buf][qq * kRowF + ch * 4 + e] = __uint_as_float(st.r[4 + i][e]);
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void bwd_dkdv_f32_kernel(BwdArgs a) {
-  __shared__ KvLdsF32 lds;
+__global__ __launch_bounds__(64 * kKvWaves) __attribute__((amdgpu_waves_per_eu(2)))
+void bwd_dkdv_f32_kernel(BwdArgs a) {
+  __shared__ F32Tile qt[kKvWaves], gt[kKvWaves];  // the waves' Q and dO blocks
+  __shared__ F32Tile kt, vt;
+  __shared__ float rows[kKvWaves][2][32];        // per wave: lse2 and -D of the block's queries
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int half = lane >> 5;
-  // 1-D grid: (key-tile item in launch order, kvh), heads fastest
-  const int slot = uniform(fast_div(blockIdx.x, a.div_hkv));
-  const int kvh = uniform(blockIdx.x - slot * a.Hkv);
-  const int item = ld_const(a.korder, slot);  // (row, key tile), longest first
-  const int b = uniform(fast_div(item, a.div_nk));
-  const int kt = uniform(item - b * a.nk);
-  const int kpos = kt * kTile + wave * 32 + (lane & 31);
+  const int wave = uniform(threadIdx.x >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  F32Unit w;
+  if (!f32_unit(a.korder, a.div_hkv, a.div_hkv, a.div_nk, a.S, 1, w)) return;
+  const int b = w.b, k0 = w.row0, kvh = w.kvh;
+  const int kpos = k0 + col;
   const int mykid = a.kid[(size_t)b * a.tk_pad + kpos];
-  const bool kvalid = kpos < a.S;
-
-  // K, V as B operands of S = Q K^T and dP = dO V^T
-  float kf[32], vf[32];
-  {
-    const size_t row = (((size_t)b * a.S + kpos) * a.Hkv + kvh) * kD;
-    const float* ks = reinterpret_cast<const float*>(a.k) + row + half;
-    const float* vs = reinterpret_cast<const float*>(a.v) + row + half;
-#pragma unroll
-    for (int st = 0; st < 32; ++st) {
-      kf[st] = kvalid ? ks[2 * st] : 0.f;
-      vf[st] = kvalid ? vs[2 * st] : 0.f;
-    }
-  }
-
-  f32x16 dkacc[2], dvacc[2];
-  dkacc[0] = dkacc[1] = dvacc[0] = dvacc[1] = zero16();
-
-  const int count = ld_const(a.kcnt, b * a.nk + kt);
-  const int* list = a.klist + ((size_t)b * a.nk + kt) * 2 * a.nq;
-  const int niters = count * a.G;  // (64-query stage, head) iterations
-  const float c = a.scale_log2;
-
-  KvStageF32 stage;
-  if (niters > 0) {
-    int qb, hg, cls;
-    kv_iter(a, list, 0, qb, hg, cls);
-    kv_load_f32(a, b, kvh * a.G + hg, qb, stage);
-    kv_store_f32(stage, lds, 0);
+  const int u = uniform(mykid);
+  const bool kuni = __all(mykid == u);
+  constexpr size_t kRow = kD * sizeof(float);
+  const size_t kv_off = ((size_t)b * a.S * a.Hkv + kvh) * kRow;
+  const uint32_t kv_stride = (uint32_t)(a.Hkv * kRow);
+  if (wave < 2) {
+    f32x4 x[8];
+    f32_load(reinterpret_cast<const char*>(wave ? a.v : a.k) + kv_off, kv_stride, k0, a.S - 1,
+             lane, x);
+    f32_store(wave ? vt : kt, lane, x);
   }
   __syncthreads();
 
-  for (int it = 0; it < niters; ++it) {
-    const int buf = it & 1;
-    int qb, hg, cls;
-    kv_iter(a, list, it, qb, hg, cls);
-    const bool partial = cls == 1;
-    if (it + 1 < niters) {
-      int qb2, hg2, cls2;
-      kv_iter(a, list, it + 1, qb2, hg2, cls2);
-      kv_load_f32(a, b, kvh * a.G + hg2, qb2, stage);
+  f32x16 dkacc[2] = {zero16(), zero16()}, dvacc[2] = {zero16(), zero16()};
+  const float c = a.scale_log2;
+  const int* list = a.klist + ((size_t)b * a.nk + w.tile) * 2 * a.nq;
+  const int niters = 2 * ld_const(a.kcnt, b * a.nk + w.tile) * a.G;  // (32-query block, head) pairs
+  const int* qid_row = a.qid + (size_t)b * a.tq_pad;
+  const uint32_t q_stride = (uint32_t)(a.Hq * kRow);
+  const char* qg = reinterpret_cast<const char*>(a.q) + (size_t)b * a.T * q_stride;
+  const char* gg = reinterpret_cast<const char*>(a.dout) + (size_t)b * a.T * q_stride;
+
+  f32x4 qx[8], gx[8];
+  int qidl = 0, entry = 0, q0 = 0, head = 0;
+  float rowl = 0.f;  // lse2 (lanes of half 0) or -D (half 1) of row q0 + col
+  // the next pair at or after `it` (in steps of 4) that is not wholly before
+  // the keys, and its rows; -1 past the list
+  auto fetch = [&](int it) {
+    for (; it < niters; it += kKvWaves) {
+      const int blk = uniform(fast_div(it, a.div_g));
+      entry = ld_const(list, blk >> 1);
+      q0 = (entry >> 2) * kStep + (blk & 1) * 32;
+      head = kvh * a.G + (it - blk * a.G);
+      if (q0 < a.T && !(a.causal && k0 > q0 + 31)) break;
     }
-
-#pragma unroll
-    for (int qb2 = 0; qb2 < 2; ++qb2) {
-      f32x16 s = zero16(), dp = zero16();
-      const float* qrow = &lds.q[buf][(qb2 * 32 + (lane & 31)) * kRowF + half];
-      const float* grow = &lds.g[buf][(qb2 * 32 + (lane & 31)) * kRowF + half];
-#pragma unroll
-      for (int st = 0; st < 32; ++st) {
-        s = mfma32x32x2(qrow[2 * st], kf[st], s);
-        dp = mfma32x32x2(grow[2 * st], vf[st], dp);
+    if (it >= niters) return -1;
+    qidl = qid_row[q0 + col];
+    f32_load(qg + head * kRow, q_stride, q0, a.T - 1, lane, qx);
+    f32_load(gg + head * kRow, q_stride, q0, a.T - 1, lane, gx);
+    // a row past the end re-reads row T - 1: its id is 0, so its pairs are
+    // masked or belong to an inactive key
+    const size_t row = ((size_t)b * a.Hq + head) * a.T;
+    const uint32_t at = 4u * (uint32_t)min(q0 + col, a.T - 1);
+    const float l2 = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.lse2 + row) + at);
+    const float nd = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.ndelta + row) + at);
+    rowl = half ? nd : l2;
+    return it;
+  };
+  int it = fetch(wave);
+  while (it >= 0) {
+    const int qb = q0;
+    bool run = true, mask_ids = false, diag = false;
+    if ((entry & 3) == 1) {
+      diag = a.causal && k0 + 31 > qb;
+      mask_ids = true;
+      if (kuni) {
+        const uint64_t same = __ballot(qidl == u);
+        run = u != 0 && same != 0;
+        mask_ids = same != ~0ull;
       }
-      // rows of s/dp are queries qq = qb2*32 + acc_row(r, lane); column = my key
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int qq0 = qb2 * 32 + 8 * g4 + 4 * half;
-        const float4 l4 = *reinterpret_cast<const float4*>(&lds.lse2[buf][qq0]);
-        const float4 d4 = *reinterpret_cast<const float4*>(&lds.dlt[buf][qq0]);
-        const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
-        const float dv4[4] = {d4.x, d4.y, d4.z, d4.w};
-        bool ok[4] = {true, true, true, true};
-        if (partial) {
-          const int4 ids = *reinterpret_cast<const int4*>(&lds.qid[buf][qq0]);
-          const int iv[4] = {ids.x, ids.y, ids.z, ids.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) ok[i] = iv[i] == mykid && (!a.causal || kpos <= qb + qq0 + i);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = g4 * 4 + i;
-          const float p = ok[i] ? fast_exp2(fmaf(s[r], c, -lv[i])) : 0.f;
-          s[r] = p;
-          dp[r] = p * (dp[r] - dv4[i]);
-        }
-      }
-#pragma unroll
-      for (int db = 0; db < 2; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int qq = qb2 * 32 + acc_row(r, lane);
-          dvacc[db] = mfma32x32x2(lds.g[buf][qq * kRowF + db * 32 + (lane & 31)], s[r], dvacc[db]);
-          dkacc[db] = mfma32x32x2(lds.q[buf][qq * kRowF + db * 32 + (lane & 31)], dp[r], dkacc[db]);
-        }
     }
-
-    if (it + 1 < niters) kv_store_f32(stage, lds, buf ^ 1);
-    __syncthreads();
-  }
-
-  if (!kvalid) return;
-  const bool kactive = mykid != 0;
-#pragma unroll
-  for (int db = 0; db < 2; ++db)
+    if (!run) {
+      it = fetch(it + kKvWaves);
+      continue;
+    }
+    wave_lds_fence();
+    rows[wave][half][col] = rowl;
+    f32_store(qt[wave], lane, qx);
+    f32_store(gt[wave], lane, gx);
+    wave_lds_fence();
+    it = fetch(it + kKvWaves);
+    f32x16 s = zero16(), dp;
+    auto row4 = [&](int which, int g4) {
+      return *reinterpret_cast<const f32x4*>(&rows[wave][which][8 * g4 + 4 * half]);
+    };
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
-      const int d0 = db * 32 + 8 * g4 + 4 * half;
-      const size_t off = (((size_t)b * a.S + kpos) * a.Hkv + kvh) * kD + d0;
-      f32x4 ok, ov;
+      const f32x4 d4 = row4(1, g4);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        ok[i] = kactive ? dkacc[db][g4 * 4 + i] * a.scale : 0.f;
-        ov[i] = kactive ? dvacc[db][g4 * 4 + i] : 0.f;
-      }
-      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.dk) + off) = ok;
-      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.dv) + off) = ov;
+      for (int e = 0; e < 4; ++e) dp[g4 * 4 + e] = d4[e];
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const f32x4 kr = kt.row4(lane, j), qr = qt[wave].row4(lane, j);
+      const f32x4 vr = vt.row4(lane, j), gr = gt[wave].row4(lane, j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s = mfma32x32x2(qr[e], kr[e], s);
+        dp = mfma32x32x2(gr[e], vr[e], dp);
+      }
+    }
+    if (mask_ids) {
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int4 ids = *reinterpret_cast<const int4*>(&qid_row[qb + 8 * g4 + 4 * half]);
+        const int iv[4] = {ids.x, ids.y, ids.z, ids.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[g4 * 4 + e] = iv[e] == mykid ? s[g4 * 4 + e] : kNegInf;
+      }
+    }
+    if (diag) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = kpos <= qb + acc_row(r, lane) ? s[r] : kNegInf;
+    }
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const f32x4 l4 = row4(0, g4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = g4 * 4 + e;
+        s[r] = fast_exp2(fmaf(s[r], c, -l4[e]));
+        dp[r] *= s[r];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        dvacc[db] = mfma32x32x2(gt[wave].col(lane, db, r), s[r], dvacc[db]);
+        dkacc[db] = mfma32x32x2(qt[wave].col(lane, db, r), dp[r], dkacc[db]);
+      }
+  }
+
+  const int etid = 64 * wave + fresh_lane_id();  // (not kept across the loop)
+  const int ek = etid / (2 * kKvWaves), d0 = kKvDims * (etid % (2 * kKvWaves));
+  const bool in = k0 + ek < a.S;
+  const bool keep = a.kid[(size_t)b * a.tk_pad + k0 + ek] != 0;
+  const size_t off = kv_off + (size_t)(k0 + ek) * kv_stride + d0 * sizeof(float);
+  auto store = [&](void* dst, const F32Tile (&t)[kKvWaves], float mul) {
+    if (!in) return;
+#pragma unroll
+    for (int h = 0; h < kKvDims / 4; ++h) {
+      f32x4 o = f32_sum(t, ek, d0 + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = keep ? o[e] * mul : 0.f;
+      *reinterpret_cast<f32x4*>(reinterpret_cast<char*>(dst) + off + 16 * h) = o;
+    }
+  };
+  wave_lds_fence();
+  f32_put(qt[wave], etid & 63, dkacc);
+  f32_put(gt[wave], etid & 63, dvacc);
+  __syncthreads();
+  store(a.dk, qt, a.scale);
+  store(a.dv, gt, 1.f);
 }
 
 // ---------------------------------------------------------------------------
@@ -1035,12 +988,13 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   a.div_hkv = make_fastdiv(a.Hkv);
   a.div_nk = make_fastdiv(a.nk);
   a.div_g = make_fastdiv(a.G);
+  a.div_hq = make_fastdiv(Hq);
   const size_t rows = (size_t)batch * T * Hq;
   const unsigned dgrid = (unsigned)((rows + 255) / 256);
-  // bf16 with both the delta and the dq phase: the dq kernel, which holds
-  // the dO rows of its queries in registers anyway, also loads O and writes
-  // D; the separate delta pass (a full read of O and dO) is skipped
-  a.fuse_delta = !f32 && (phases & 3) == 3;
+  // with both the delta and the dq phase the dq kernel, which holds the dO
+  // rows of its queries in registers anyway, also loads O and writes D; the
+  // separate delta pass (a full read of O and dO) is skipped
+  a.fuse_delta = (phases & 3) == 3;
   if ((phases & 1) && !a.fuse_delta) {
     if (f32)
       hipLaunchKernelGGL((bwd_delta_kernel<true>), dim3(dgrid), dim3(256), 0, stream, a, batch);
@@ -1050,10 +1004,7 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   const dim3 qgrid(Hkv * a.hchunks * batch * lay.nq);
   if (!(phases & 2)) {
   } else if (f32) {
-    if (hpw == 2)
-      hipLaunchKernelGGL((bwd_dq_f32_kernel<2>), qgrid, dim3(256), 0, stream, a);
-    else
-      hipLaunchKernelGGL((bwd_dq_f32_kernel<1>), qgrid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(bwd_dq_f32_kernel, dim3(4 * Hq * batch * lay.nq), dim3(256), 0, stream, a);
   } else {
     if (hpw == 2)
       hipLaunchKernelGGL((bwd_dq_bf16_kernel<2>), qgrid, dim3(512), 0, stream, a);
@@ -1066,7 +1017,7 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
     // C2/C3/C5 than 8-wave workgroups whose halves took different heads and
     // summed through LDS, because the workgroups of a CU share no barriers.
     if (f32)
-      hipLaunchKernelGGL(bwd_dkdv_f32_kernel, kgrid, dim3(256), 0, stream, a);
+      hipLaunchKernelGGL(bwd_dkdv_f32_kernel, dim3(4 * Hkv * batch * lay.nk), dim3(64 * kKvWaves), 0, stream, a);
     else
       hipLaunchKernelGGL(bwd_dkdv_bf16_kernel, kgrid, dim3(256), 0, stream, a);
   }

@@ -1,20 +1,17 @@
 // Flash-style forward for segment-masked GQA attention on gfx950.
 //
 // Two kernels: the bf16 one (further below; the benchmarked path) and an
-// fp32 one.  fp32 work unit: one workgroup = 4 waves = one 128-query
-// tile of one row, for HPW (1 or 2) query heads that share a KV head.  Each
-// wave owns 32 queries for all HPW heads, so every K / V^T fragment it reads
-// from LDS feeds HPW MFMAs (the GQA sharing of K/V tiles).  The workgroup
-// walks the compacted list of non-empty 128-key tiles of its query tile (from
-// the block map) in 64-key steps, double-buffering K and V in LDS.
+// fp32 one.  Both walk the compacted list of non-empty 64-key stages of a
+// 128-query tile (from the block map).
 //
 // Scores are formed transposed, S^T = K Q^T, so an accumulator column is one
 // query: the row max and row sum are in-lane reductions plus one
 // v_permlane32_swap, and the exponentiated block is already in the register
-// layout of the B operand of O^T += V^T P^T.  PARTIAL tiles compare the
-// canonical ids (and causality) per element; FULL tiles skip the compare.
+// layout of the B operand of O^T += V^T P^T.  PARTIAL stages compare the
+// canonical ids (and causality) per element; FULL stages skip the compare.
 // Online softmax in base 2 with the logit scale folded into one FMA.
 #include "mf_common.h"
+#include "mf_f32.h"
 #include "mf_lds.h"
 
 namespace mf {
@@ -35,6 +32,7 @@ struct FwdArgs {
   int causal;
   float scale, scale_log2;
   FastDiv div_nh, div_hchunks, div_nq;  // Hkv * hchunks, hchunks, nq
+  FastDiv div_hq, div_hkv;              // Hq, Hkv (fp32 units)
   // query prologue fused into the bf16 kernel's query loads (ROPE instances)
   const void* q_gain;           // [64], tensor dtype
   const int32_t* positions;     // [B, T] or null (0 .. T-1 on every row)
@@ -44,220 +42,177 @@ struct FwdArgs {
 };
 
 constexpr int kStepK = 64;          // keys per inner step
-constexpr int kLdsRowF = kD + 1;    // fp32 LDS row pitch (65 floats)
 
-struct FwdLdsF32 {
-  float k[2][kStepK * kLdsRowF];  // K [key][d]
-  float v[2][kStepK * kLdsRowF];  // V [key][d]
-  int kid[2][kStepK];
-};
-
-// Global -> register staging of one 64-key step (K and V) for the workgroup.
-struct FwdStageF32 {
-  u32x4 r[8];
-};
-
-__device__ __forceinline__ void fwd_load_f32(const FwdArgs& a, int b, int kvh, int kb,
-                                             FwdStageF32& st) {
-  const int tid = threadIdx.x;
-  const float* ks = reinterpret_cast<const float*>(a.k);
-  const float* vs = reinterpret_cast<const float*>(a.v);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = tid + 256 * i;
-    const int key = kb + (u >> 4), ch = u & 15;
-    const size_t off = (((size_t)b * a.S + key) * a.Hkv + kvh) * kD + ch * 4;
-    st.r[i] = key < a.S ? ld_u32x4(ks + off) : u32x4{0, 0, 0, 0};
-    st.r[4 + i] = key < a.S ? ld_u32x4(vs + off) : u32x4{0, 0, 0, 0};
-  }
-}
-
-__device__ __forceinline__ void fwd_store_f32(const FwdArgs& a, int b, int kb,
-                                              const FwdStageF32& st, FwdLdsF32& lds, int buf) {
-  const int tid = threadIdx.x;
-  if (tid < kStepK) lds.kid[buf][tid] = a.kid[(size_t)b * a.tk_pad + kb + tid];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = tid + 256 * i;
-    const int key = u >> 4, ch = u & 15;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      lds.k[buf][key * kLdsRowF + ch * 4 + e] = __uint_as_float(st.r[i][e]);
-      lds.v[buf][key * kLdsRowF + ch * 4 + e] = __uint_as_float(st.r[4 + i][e]);
-    }
-  }
-}
-
-template <int HPW>
-__global__ __launch_bounds__(256) void attn_fwd_f32_kernel(FwdArgs a) {
-  __shared__ FwdLdsF32 lds;
+// ---------------------------------------------------------------------------
+// fp32 forward: one workgroup per (32-query block, query head); its four
+// waves take every fourth 32-key block of the tile's work list and merge
+// their softmax states through LDS at the end (fixed wave order).
+//
+// Bound: v_mfma_f32_32x32x2_f32, 64 cycles each and 64 of them per 32x32
+// block, one dependent chain per wave.  A 128-query x 2-head workgroup (the
+// bf16 kernel's shape) leaves the chip idle at the sizes fp32 is used at and
+// makes each wave walk the whole list twice over; splitting queries, heads
+// and keys gives 16 times the workgroups with a chain an eighth as long, and
+// skips the 32x32 blocks no pair of which is valid.  Measured (same box, us
+// per launch, before -> after): 2 x 256 tokens, 4/2 heads, segments 1-64:
+// 42.5 -> 10.5; 2 x 1499, 16/8 heads, causal, mean segment 512: 105 -> 29.7.
+// Each wave stages its own K and V blocks (its keys are nobody else's), the
+// next block's rows in flight while it works on this one's.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void attn_fwd_f32_kernel(FwdArgs a) {
+  __shared__ F32Tile kt[4], vt[4], qt;  // the waves' K and V blocks; the queries
+  __shared__ float lm[4][32], ll[4][32];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int half = lane >> 5;
-  // 1-D grid: (query-tile item in launch order, kvh, head chunk), heads fastest
-  const int nh = a.Hkv * a.hchunks;
-  const int slot = uniform(fast_div(blockIdx.x, a.div_nh));
-  const int hr = uniform(blockIdx.x - slot * nh);
-  const int kvh = uniform(fast_div(hr, a.div_hchunks));
-  const int hc = uniform(hr - kvh * a.hchunks);
-  const int item = ld_const(a.qorder, slot);  // (row, query tile), longest first
-  const int b = uniform(fast_div(item, a.div_nq));
-  const int qt = uniform(item - b * a.nq);
-  const int qpos = qt * kTile + wave * 32 + (lane & 31);
+  const int wave = uniform(threadIdx.x >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  F32Unit w;
+  if (!f32_unit(a.qorder, a.div_hq, a.div_hkv, a.div_nq, a.T, a.G, w)) return;
+  const int b = w.b, q0 = w.row0, kvh = w.kvh, head = w.head;
+  const int qpos = q0 + col;
   const int myqid = a.qid[(size_t)b * a.tq_pad + qpos];
-  const bool qvalid = qpos < a.T;
-  int head[HPW];
-#pragma unroll
-  for (int j = 0; j < HPW; ++j) head[j] = kvh * a.G + hc * HPW + j;
+  const int u = uniform(myqid);
+  const bool quni = __all(myqid == u);
 
-  // ---- query fragments (B operand of S^T = K Q^T) -----------------------
-  float qf[HPW][32];
-#pragma unroll
-  for (int j = 0; j < HPW; ++j) {
-    const float* src = reinterpret_cast<const float*>(a.q) +
-                       (((size_t)b * a.T + qpos) * a.Hq + head[j]) * kD + half;
-#pragma unroll
-    for (int st = 0; st < 32; ++st) qf[j][st] = qvalid ? src[2 * st] : 0.f;
+  constexpr size_t kRow = kD * sizeof(float);
+  if (wave == 0) {
+    f32x4 x[8];
+    f32_load(reinterpret_cast<const char*>(a.q) + ((size_t)b * a.T * a.Hq + head) * kRow,
+             (uint32_t)(a.Hq * kRow), q0, a.T - 1, lane, x);
+    f32_store(qt, lane, x);
   }
 
-  f32x16 oacc[HPW][2];
-  float m[HPW], l[HPW];
-#pragma unroll
-  for (int j = 0; j < HPW; ++j) {
-    oacc[j][0] = zero16();
-    oacc[j][1] = zero16();
-    m[j] = kNegInf;
-    l[j] = 0.f;
-  }
-
-  const int count = ld_const(a.qcnt, b * a.nq + qt);
-  const int* list = a.qlist + ((size_t)b * a.nq + qt) * 2 * a.nk;
-  const int nsteps = count;  // one 64-key stage per list entry
+  f32x16 oacc[2] = {zero16(), zero16()};
+  float m = kNegInf, l = 0.f;
   const float c = a.scale_log2;
+  const int* list = a.qlist + ((size_t)b * a.nq + w.tile) * 2 * a.nk;
+  const int nb = 2 * ld_const(a.qcnt, b * a.nq + w.tile);  // 32-key blocks
+  const int* kid_row = a.kid + (size_t)b * a.tk_pad;
+  const char* kg = reinterpret_cast<const char*>(a.k) + ((size_t)b * a.S * a.Hkv + kvh) * kRow;
+  const char* vg = reinterpret_cast<const char*>(a.v) + ((size_t)b * a.S * a.Hkv + kvh) * kRow;
+  const uint32_t kv_stride = (uint32_t)(a.Hkv * kRow);
 
-  FwdStageF32 stage;
-  if (nsteps > 0) {
-    const int e0 = list[0];
-    fwd_load_f32(a, b, kvh, (e0 >> 2) * kStepK, stage);
-    fwd_store_f32(a, b, (e0 >> 2) * kStepK, stage, lds, 0);
-  }
+  f32x4 kx[8], vx[8];
+  int kidl = 0, entry = 0, k0 = 0;
+  // block i's rows; false past the list or, when causal, past the
+  // queries (stages ascend, so every later block is past them too)
+  auto fetch = [&](int i) {
+    if (i >= nb) return false;
+    entry = ld_const(list, i >> 1);
+    k0 = (entry >> 2) * kStepK + (i & 1) * 32;
+    if (a.causal && k0 > q0 + 31) return false;
+    kidl = kid_row[k0 + col];
+    f32_load(kg, kv_stride, k0, a.S - 1, lane, kx);
+    f32_load(vg, kv_stride, k0, a.S - 1, lane, vx);
+    return true;
+  };
+  int i = wave;
+  bool more = fetch(i);
   __syncthreads();
-
-  for (int step = 0; step < nsteps; ++step) {
-    const int buf = step & 1;
-    const int entry = list[step];
-    const int kb = (entry >> 2) * kStepK;
-    const bool partial = (entry & 3) == 1;
-    int next_kb = 0;
-    if (step + 1 < nsteps) {
-      next_kb = (list[step + 1] >> 2) * kStepK;
-      fwd_load_f32(a, b, kvh, next_kb, stage);
-    }
-
-    // ---- S^T = K Q^T for two 32-key blocks --------------------------------
-    f32x16 s[HPW][2];
-#pragma unroll
-    for (int kb2 = 0; kb2 < 2; ++kb2) {
-#pragma unroll
-      for (int j = 0; j < HPW; ++j) s[j][kb2] = zero16();
-      const float* krow = &lds.k[buf][(kb2 * 32 + (lane & 31)) * kLdsRowF + half];
-#pragma unroll
-      for (int st = 0; st < 32; ++st) {
-        const float af = krow[2 * st];
-#pragma unroll
-        for (int j = 0; j < HPW; ++j) s[j][kb2] = mfma32x32x2(af, qf[j][st], s[j][kb2]);
+  while (more) {
+    const int kb = k0;
+    bool run = true, mask_ids = false, diag = false;
+    if ((entry & 3) == 1) {
+      diag = a.causal && kb + 31 > q0;
+      mask_ids = true;
+      if (quni) {
+        const uint64_t same = __ballot(kidl == u);
+        run = u != 0 && same != 0;
+        mask_ids = same != ~0ull;
       }
     }
-
-    // ---- element mask on PARTIAL tiles ------------------------------------
-    if (partial) {
+    i += 4;
+    if (!run) {
+      more = fetch(i);
+      continue;
+    }
+    wave_lds_fence();
+    f32_store(kt[wave], lane, kx);
+    f32_store(vt[wave], lane, vx);
+    wave_lds_fence();
+    more = fetch(i);
+    f32x16 s = zero16();
 #pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2) {
+    for (int j = 0; j < 8; ++j) {
+      const f32x4 kr = kt[wave].row4(lane, j), qr = qt.row4(lane, j);
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int kk0 = kb2 * 32 + 8 * g4 + 4 * half;
-          const int4 kids = *reinterpret_cast<const int4*>(&lds.kid[buf][kk0]);
-          const int kv[4] = {kids.x, kids.y, kids.z, kids.w};
+      for (int e = 0; e < 4; ++e) s = mfma32x32x2(kr[e], qr[e], s);
+    }
+    if (mask_ids) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const bool ok = kv[i] == myqid && (!a.causal || kb + kk0 + i <= qpos);
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int4 kids = *reinterpret_cast<const int4*>(&kid_row[kb + 8 * g4 + 4 * half]);
+        const int kv[4] = {kids.x, kids.y, kids.z, kids.w};
 #pragma unroll
-            for (int j = 0; j < HPW; ++j)
-              s[j][kb2][g4 * 4 + i] = ok ? s[j][kb2][g4 * 4 + i] : kNegInf;
-          }
-        }
+        for (int e = 0; e < 4; ++e) s[g4 * 4 + e] = kv[e] == myqid ? s[g4 * 4 + e] : kNegInf;
       }
     }
-
-    // ---- online softmax (base 2) -------------------------------------------
+    if (diag) {
 #pragma unroll
-    for (int j = 0; j < HPW; ++j) {
-      float mx = kNegInf;
+      for (int r = 0; r < 16; ++r) s[r] = kb + acc_row(r, lane) <= qpos ? s[r] : kNegInf;
+    }
+    float mx = s[0];
 #pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(s[j][kb2][r], s[j][kb2][r + 1]));
-      mx = halves_max(mx);
-      const float mnew = fmaxf(m[j], mx);
-      const float msafe = mnew == kNegInf ? 0.f : mnew;
-      const float alpha = fast_exp2((m[j] - msafe) * c);
-      m[j] = mnew;
-      l[j] *= alpha;
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = halves_max(mx);
+    if (__any(mx > m)) {
+      const float mnew = fmaxf(m, mx);
+      const float alpha = mnew == kNegInf ? 1.f : fast_exp2((m - mnew) * c);
+      m = mnew;
+      l *= alpha;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        oacc[j][0][r] *= alpha;
-        oacc[j][1][r] *= alpha;
+        oacc[0][r] *= alpha;
+        oacc[1][r] *= alpha;
       }
-      const float mc = msafe * c;
-#pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = fast_exp2(fmaf(s[j][kb2][r], c, -mc));
-          s[j][kb2][r] = p;
-          l[j] += p;
-        }
     }
-
-    // ---- O^T += V^T P^T -------------------------------------------------------
+    const float mc = m == kNegInf ? 0.f : m * c;
 #pragma unroll
-    for (int db = 0; db < 2; ++db)
+    for (int r = 0; r < 16; ++r) {
+      s[r] = fast_exp2(fmaf(s[r], c, -mc));
+      l += s[r];
+    }
 #pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float vf = lds.v[buf][(kb2 * 32 + acc_row(r, lane)) * kLdsRowF + db * 32 + (lane & 31)];
-#pragma unroll
-          for (int j = 0; j < HPW; ++j) oacc[j][db] = mfma32x32x2(vf, s[j][kb2][r], oacc[j][db]);
-        }
-
-    if (step + 1 < nsteps) fwd_store_f32(a, b, next_kb, stage, lds, buf ^ 1);
-    __syncthreads();
+    for (int r = 0; r < 16; ++r) {
+      oacc[0] = mfma32x32x2(vt[wave].col(lane, 0, r), s[r], oacc[0]);
+      oacc[1] = mfma32x32x2(vt[wave].col(lane, 1, r), s[r], oacc[1]);
+    }
   }
 
-  // ---- epilogue ----------------------------------------------------------------
-  const bool qactive = qvalid && myqid != 0;
+  // merge the waves' (max, sum, O): thread = (query, 8 dims)
+  l = halves_sum(l);
+  if (half == 0) {
+    lm[wave][col] = m;
+    ll[wave][col] = l;
+  }
+  wave_lds_fence();
+  f32_put(kt[wave], lane, oacc);
+  __syncthreads();
+  const int eq = threadIdx.x >> 3, d0 = 8 * (threadIdx.x & 7);
+  const int eqpos = q0 + eq;
+  if (eqpos >= a.T) return;
+  float M = lm[0][eq];
 #pragma unroll
-  for (int j = 0; j < HPW; ++j) {
-    const float lt = halves_sum(l[j]);
-    const bool has = qactive && lt > 0.f;
-    const float inv = has ? 1.f / lt : 0.f;
-    if (qvalid) {
-      if (half == 0)
-        a.lse[((size_t)b * a.Hq + head[j]) * a.T + qpos] =
-            has ? fmaf(m[j], a.scale, __logf(lt)) : kPosInf;
+  for (int x = 1; x < 4; ++x) M = fmaxf(M, lm[x][eq]);
+  float wt[4], lt = 0.f;
 #pragma unroll
-      for (int db = 0; db < 2; ++db)
+  for (int x = 0; x < 4; ++x) {
+    wt[x] = M == kNegInf ? 0.f : fast_exp2((lm[x][eq] - M) * c);
+    lt = fmaf(wt[x], ll[x][eq], lt);
+  }
+  const bool has = a.qid[(size_t)b * a.tq_pad + eqpos] != 0 && lt > 0.f;
+  const float inv = has ? 1.f / lt : 0.f;
+  if ((threadIdx.x & 7) == 0)
+    a.lse[((size_t)b * a.Hq + head) * a.T + eqpos] = has ? fmaf(M, a.scale, __logf(lt)) : kPosInf;
+  float* dst = reinterpret_cast<float*>(a.out) + (((size_t)b * a.T + eqpos) * a.Hq + head) * kD + d0;
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int d0 = db * 32 + 8 * g4 + 4 * half;
-          const size_t off = (((size_t)b * a.T + qpos) * a.Hq + head[j]) * kD + d0;
-          f32x4 o;
+  for (int h = 0; h < 2; ++h) {
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = has ? oacc[j][db][g4 * 4 + i] * inv : 0.f;
-          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + off) = o;
-        }
-    }
+    for (int x = 0; x < 4; ++x) o += f32_at(kt[x], eq, d0 + 4 * h) * wt[x];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = has ? o[e] * inv : 0.f;
+    *reinterpret_cast<f32x4*>(dst + 4 * h) = o;
   }
 }
 
@@ -640,6 +595,8 @@ static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, 
   a.div_nh = make_fastdiv(a.Hkv * a.hchunks);
   a.div_hchunks = make_fastdiv(a.hchunks);
   a.div_nq = make_fastdiv(a.nq);
+  a.div_hq = make_fastdiv(Hq);
+  a.div_hkv = make_fastdiv(Hkv);
   return a;
 }
 
@@ -650,10 +607,7 @@ hipError_t launch_attn_fwd(const void* q, const void* k, const void* v, bool f32
   const FwdArgs a = fwd_args(q, k, v, batch, T, S, Hq, Hkv, mode, scale, plan, out, lse, &hpw);
   const dim3 grid(Hkv * a.hchunks * batch * a.nq);
   if (f32) {
-    if (hpw == 2)
-      hipLaunchKernelGGL((attn_fwd_f32_kernel<2>), grid, dim3(256), 0, stream, a);
-    else
-      hipLaunchKernelGGL((attn_fwd_f32_kernel<1>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(4 * Hq * batch * a.nq), dim3(256), 0, stream, a);
   } else {
     if (hpw == 2)
       hipLaunchKernelGGL((attn_fwd_bf16_kernel<2, false>), grid, dim3(512), 0, stream, a);
