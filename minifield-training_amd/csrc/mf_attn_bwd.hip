@@ -428,16 +428,16 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
 
 // ---------------------------------------------------------------------------
 // bf16 dq: the structure of the bf16 forward (one head per wave, 4*HPW
-// waves, K/V tiles DMA'd into a two-slot LDS ring of 128-key slots).
+// waves, K/V tiles DMA'd into a two-slot LDS ring).
 // dQ^T += K^T dS^T takes its K^T operand from the K tile through
 // transposing LDS reads.
 // ---------------------------------------------------------------------------
 template <int HPW>
-__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(2 * HPW)))
+__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(HPW + 2)))
 void bwd_dq_bf16_kernel(BwdArgs a) {
   constexpr int W = 4 * HPW;
-  // two ring slots of 128 keys, each two 64-key stages
-  __shared__ __attribute__((aligned(16))) char slotA[2 * kStageBytes], slotB[2 * kStageBytes];
+  constexpr int SLOT = HPW;  // 64-key stages per ring slot
+  __shared__ __attribute__((aligned(16))) char slotA[SLOT * kStageBytes], slotB[SLOT * kStageBytes];
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   const int half = lane >> 5;
@@ -569,14 +569,14 @@ void bwd_dq_bf16_kernel(BwdArgs a) {
     }
   };
 
-  // Ring of two 128-key slots (as in the forward): slot i+1's DMAs are issued
-  // right after the barrier that opens slot i; whole pairs of slots, with the
+  // Ring of two slots (as in the forward): slot i+1's DMAs are issued right
+  // after the barrier that opens slot i; whole pairs of slots, with the
   // computes past the end skipped.
   auto issue_slot = [&](int i, int e0, int e1, char* slot) {
-    if (2 * i < nsteps) issue(e0, slot);
-    if (2 * i + 1 < nsteps) issue(e1, slot + kStageBytes);
+    if (SLOT * i < nsteps) issue(e0, slot);
+    if (SLOT == 2 && 2 * i + 1 < nsteps) issue(e1, slot + kStageBytes);
   };
-  const int nslots = (nsteps + 1) >> 1;
+  const int nslots = SLOT == 2 ? (nsteps + 1) >> 1 : nsteps;
   // Both slots and the query-side rows (q, dO, lse, O for D) are in flight
   // together before the first wait; after that slot i+1's DMAs are issued
   // when slot i opens.  The list entries a pair of slots needs (steps
@@ -587,7 +587,7 @@ void bwd_dq_bf16_kernel(BwdArgs a) {
   {
     const i32x8u e = ld_const8(list, 0);
     issue_slot(0, e[0], e[1], slotA);
-    issue_slot(1, e[2], e[3], slotB);
+    issue_slot(1, e[SLOT], e[SLOT + 1], slotB);
   }
   {
     const size_t row = (((size_t)b * a.T + min(qpos, a.T - 1)) * a.Hq + head) * kD + 8 * half;
@@ -633,18 +633,18 @@ void bwd_dq_bf16_kernel(BwdArgs a) {
   }
   // (a slot past the end is skipped whole, as in the forward)
   for (int i = 0; i < nslots; i += 2) {
-    const i32x8u e = ld_const8(list, 2 * i);
+    const i32x8u e = ld_const8(list, SLOT * i);
     wait_vmcnt<0>();
     barrier();
-    if (i > 0) issue_slot(i + 1, e[2], e[3], slotB);
+    if (i > 0) issue_slot(i + 1, e[SLOT], e[SLOT + 1], slotB);
     compute(e[0], slotA);
-    if (2 * i + 1 < nsteps) compute(e[1], slotA + kStageBytes);
+    if (SLOT == 2 && 2 * i + 1 < nsteps) compute(e[1], slotA + kStageBytes);
     if (i + 1 < nslots) {
       wait_vmcnt<0>();
       barrier();
-      issue_slot(i + 2, e[4], e[5], slotA);
-      compute(e[2], slotB);
-      if (2 * i + 3 < nsteps) compute(e[3], slotB + kStageBytes);
+      issue_slot(i + 2, e[2 * SLOT], e[2 * SLOT + 1], slotA);
+      compute(e[SLOT], slotB);
+      if (SLOT == 2 && 2 * i + 3 < nsteps) compute(e[3], slotB + kStageBytes);
     }
   }
   wait_vmcnt<0>();
@@ -973,6 +973,12 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   a.Hq = Hq;
   a.Hkv = Hkv;
   a.G = Hq / Hkv;
+  // dq: two heads per workgroup where the group splits into pairs; one, with
+  // one-stage ring slots (three workgroups per CU at 132 VGPRs), for odd
+  // groups (8 x 4096, segments 32-2048, 12/4 heads: 156 us against 170 with
+  // two-stage slots, 8/8: 104 against 112).  Small even calls keep two heads:
+  // one measured 24 us against 20.5 at 1 x 8192 of short segments and -6 to
+  // +5% at others.
   const int hpw = (a.G % 2 == 0) ? 2 : 1;
   a.hchunks = a.G / hpw;
   a.nq = lay.nq;

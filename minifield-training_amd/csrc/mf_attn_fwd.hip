@@ -229,6 +229,12 @@ void attn_fwd_f32_kernel(FwdArgs a) {
 // it by more than 8 in log2 units, so P <= 2^8 and the final division by the
 // row sum is unchanged.  Row sums are v_dot2 of the bf16 probabilities with
 // (1, 1), a full-rate VALU op that halves the adds.
+//
+// A workgroup serves HPW heads, four waves each.  Two heads share every K/V
+// stage and win where the chip is full.  One head takes ring slots of one
+// stage (33 KB of LDS, so four workgroups fit a CU, as two two-head ones do)
+// and is the finer unit; a wave's arithmetic, and so every output bit, is the
+// same.  heads_per_block has the rule and what both measure.
 // ---------------------------------------------------------------------------
 // The query half of the attention prologue on the query fragments a lane
 // holds (dims 16 ks + 8 half .. +7 of one query row, ks = 0..3; the other
@@ -311,11 +317,11 @@ __device__ __forceinline__ void rope_query(const FwdArgs& a, int b, int qpos, in
 }
 
 template <int HPW, bool ROPE>
-__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(2 * HPW)))
+__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(4)))
 void attn_fwd_bf16_kernel(FwdArgs a) {
   constexpr int W = 4 * HPW;
-  // two ring slots of 128 keys, each two 64-key stages
-  __shared__ __attribute__((aligned(16))) char slotA[2 * kStageBytes], slotB[2 * kStageBytes];
+  constexpr int SLOT = HPW;  // 64-key stages per ring slot
+  __shared__ __attribute__((aligned(16))) char slotA[SLOT * kStageBytes], slotB[SLOT * kStageBytes];
   const int lane = threadIdx.x & 63;
   // scalar wave index: keeps the DMA destinations scalar expressions of the
   // stage arrays, so the compiler sees which stage each DMA writes
@@ -494,19 +500,19 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
     if (run[1]) finish_pv(s1, vt, 1);
   };
 
-  // Ring of two 128-key slots: the DMAs of slot i+1 are issued right after
-  // the barrier that opens slot i, so they have the compute of slot i (four
-  // 32-key blocks) to land, and one barrier serves 128 keys.
+  // Ring of two slots (two 64-key stages each with two heads, one with one):
+  // the DMAs of slot i+1 are issued right after the barrier that opens slot i,
+  // so they have the compute of slot i to land, and one barrier serves a slot.
   auto issue_slot = [&](int i, int e0, int e1, char* slot) {
-    if (2 * i < nsteps) issue(e0, slot);
-    if (2 * i + 1 < nsteps) issue(e1, slot + kStageBytes);
+    if (SLOT * i < nsteps) issue(e0, slot);
+    if (SLOT == 2 && 2 * i + 1 < nsteps) issue(e1, slot + kStageBytes);
   };
-  const int nslots = (nsteps + 1) >> 1;
-  // The list entries a pair of slots needs (steps 2i .. 2i+5) arrive in one
-  // scalar load of eight, issued before the pair's first wait.  The read may
-  // run up to 7 entries past the list's end, into the plan's next section
-  // (query lists are followed by the key-tile counts); entries at or past
-  // nsteps are never used.
+  const int nslots = SLOT == 2 ? (nsteps + 1) >> 1 : nsteps;
+  // The list entries a pair of slots needs (the pair's and the next slot's)
+  // arrive in one scalar load of eight, issued before the pair's first wait.
+  // The read may run up to 7 entries past the list's end, into the plan's next
+  // section (query lists are followed by the key-tile counts); entries at or
+  // past nsteps are never used.
   {
     const i32x8u e = ld_const8(list, 0);
     issue_slot(0, e[0], e[1], slotA);
@@ -516,18 +522,18 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
   // leaving the loop mid-pair (a mid-pair exit gives the accumulators two
   // exit paths, resolved with register copies).
   for (int i = 0; i < nslots; i += 2) {
-    const i32x8u e = ld_const8(list, 2 * i);
+    const i32x8u e = ld_const8(list, SLOT * i);
     wait_vmcnt<0>();
     barrier();
-    issue_slot(i + 1, e[2], e[3], slotB);
-    compute(2 * i, e[0], slotA);
-    if (2 * i + 1 < nsteps) compute(2 * i + 1, e[1], slotA + kStageBytes);
+    issue_slot(i + 1, e[SLOT], e[SLOT + 1], slotB);
+    compute(SLOT * i, e[0], slotA);
+    if (SLOT == 2 && 2 * i + 1 < nsteps) compute(2 * i + 1, e[1], slotA + kStageBytes);
     if (i + 1 < nslots) {
       wait_vmcnt<0>();
       barrier();
-      issue_slot(i + 2, e[4], e[5], slotA);
-      compute(2 * i + 2, e[2], slotB);
-      if (2 * i + 3 < nsteps) compute(2 * i + 3, e[3], slotB + kStageBytes);
+      issue_slot(i + 2, e[2 * SLOT], e[2 * SLOT + 1], slotA);
+      compute(SLOT * i + SLOT, e[SLOT], slotB);
+      if (SLOT == 2 && 2 * i + 3 < nsteps) compute(2 * i + 3, e[3], slotB + kStageBytes);
     }
   }
   wait_vmcnt<0>();  // no DMA may still target this workgroup's LDS at exit
@@ -559,9 +565,25 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
   }
 }
 
+// Heads per workgroup of the bf16 forward: one for odd groups and for calls
+// whose one-head workgroups are all resident at once (four on each of the 256
+// CUs), two otherwise.  us with two heads (odd groups: one head with two-stage
+// slots, two workgroups per CU) and with one:
+//   1 x 5003, one causal segment, 16/8 heads   128 -> 110    (640 workgroups)
+//   1 x 2048, mean segment 512, 16/8            19.2 -> 15.9 (256)
+//   1 x 8192, one segment, 16/8                217 -> 200    (1024)
+//   1 x 8192, segments 16-128, 16/8             17.6 -> 18.5 (1024)
+//   1 x 16384, segments 16-128, 16/8            31.5 -> 32.0 (2048: two)
+//   4 x 8192, mean segment 512, 16/8            98 -> 106    (4096: two)
+//   4 x 4096, mean segment 512, 32/8            75 -> 86     (4096: two)
+//   8 x 4096, segments 32-2048, 12/4           127 -> 104    (odd)
+//   8 x 4096, segments 32-2048, 8/8             85.5 -> 72   (odd)
+static int heads_per_block(int G, long long tile_heads) {
+  return G % 2 == 0 && tile_heads > 4 * 256 ? 2 : 1;
+}
+
 // Arguments of one forward launch: operands, the plan's sections, shapes and
-// the workgroup shape (heads per workgroup: 2 when the GQA group splits into
-// pairs, else 1).
+// the workgroup shape (heads per workgroup).
 static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, int T, int S,
                         int Hq, int Hkv, int mode, float scale, const void* plan, void* out,
                         float* lse, int* hpw) {
@@ -583,7 +605,7 @@ static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, 
   a.Hq = Hq;
   a.Hkv = Hkv;
   a.G = Hq / Hkv;
-  *hpw = (a.G % 2 == 0) ? 2 : 1;
+  *hpw = heads_per_block(a.G, (long long)batch * lay.nq * Hq);
   a.hchunks = a.G / *hpw;
   a.nq = lay.nq;
   a.nk = lay.nk;
