@@ -77,6 +77,9 @@ def packed_causal_attention(
 
 def _lengths(valid_length, batch: int, device: torch.device) -> torch.Tensor:
     if isinstance(valid_length, torch.Tensor):
+        if (valid_length.dtype is torch.int32 and valid_length.shape == (batch,)
+                and valid_length.device == device and valid_length.is_contiguous()):
+            return valid_length
         lengths = valid_length.to(device=device, dtype=torch.int32).reshape(-1)
     else:
         lengths = torch.tensor(valid_length, dtype=torch.int32, device=device).reshape(-1)

@@ -35,9 +35,10 @@ def _positions(positions, batch: int, length: int, device: torch.device) -> torc
 
 
 def _launch_forward(q, k, qg, kg, pos, eps, theta, q_out, k_out):
+    b, t, hq, d = q.shape
     _lib.check(_lib.LIB.mf_qk_norm_rope(_ptr(q), _ptr(k), _ptr(qg), _ptr(kg), _ptr(pos),
-                                        dtype_code(q), q.shape[0], q.shape[1], q.shape[2],
-                                        k.shape[2], q.shape[3], float(eps), float(theta),
+                                        dtype_code(q), b, t, hq, k.shape[2], d, float(eps),
+                                        float(theta),
                                         _ptr(q_out), _ptr(k_out), _stream(q.device)))
 
 
@@ -61,17 +62,20 @@ class QKNormRope(torch.autograd.Function):
         dq_out = torch.zeros_like(q) if dq_out is None else dq_out.contiguous()
         dk_out = torch.zeros_like(k) if dk_out is None else dk_out.contiguous()
         dq, dk = torch.empty_like(q), torch.empty_like(k)
-        dqg = torch.empty(q.shape[-1], dtype=torch.float32, device=q.device)
-        dkg = torch.empty_like(dqg)
-        b, t = q.shape[:2]
+        b, t, hq, d = q.shape
+        # both gain gradients in one buffer, cast to the gains' dtype (the
+        # tensors') by one launch
+        dgains = torch.empty((2, d), dtype=torch.float32, device=q.device)
+        dqg = dgains.data_ptr()
         ws_bytes = _lib.LIB.mf_qk_norm_rope_bwd_workspace_bytes(b, t)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
         _lib.check(_lib.LIB.mf_qk_norm_rope_bwd(
             _ptr(q), _ptr(k), _ptr(qg), _ptr(kg), _ptr(pos), _ptr(dq_out), _ptr(dk_out),
-            dtype_code(q), b, t, q.shape[2], k.shape[2], q.shape[3], float(ctx.eps),
-            float(ctx.theta), _ptr(dq), _ptr(dk), _ptr(dqg), _ptr(dkg), _ptr(ws), ws_bytes,
+            dtype_code(q), b, t, hq, k.shape[2], d, float(ctx.eps),
+            float(ctx.theta), _ptr(dq), _ptr(dk), dqg, dqg + 4 * d, _ptr(ws), ws_bytes,
             _stream(q.device)))
-        return dq, dk, dqg.to(qg.dtype), dkg.to(kg.dtype), None, None, None
+        dgains = dgains.to(qg.dtype)
+        return dq, dk, dgains[0], dgains[1], None, None, None
 
 
 def qk_norm_rope(query: torch.Tensor, key: torch.Tensor, query_gain: torch.Tensor,

@@ -20,8 +20,13 @@ from . import _lib
 _DTYPES = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
 
 
+# The current stream's handle by device index.  torch.cuda.current_stream
+# builds a Stream object for the same number (1.9 us against 0.1).
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -31,12 +36,13 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """Every operand must already live on one ROCm device (no host fallback)."""
     device = tensors[0].device
+    index = device.index
     for t in tensors:
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError(
                 "mfattn runs on the GPU only; got a tensor on " + str(t.device)
             )
-        if t.device != device:
+        if t.get_device() != index:
             raise ValueError("all operands must be on the same device")
     return device
 
@@ -62,7 +68,7 @@ def same_dtype(what: str, *tensors: torch.Tensor) -> int:
 
 
 def _require_shape(t: torch.Tensor, shape: tuple[int, ...], what: str) -> None:
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:  # torch.Size compares as a tuple
         raise ValueError(f"{what} must be {list(shape)}, got {list(t.shape)}")
 
 
@@ -98,9 +104,10 @@ def as_mask(mask: torch.Tensor, mode: int) -> tuple[torch.Tensor, int]:
     causal mode (``attention.py:97``), ``!= 0`` for the bidirectional modes
     (``bidirectional.py:22,25``).
     """
-    if mask.dtype == torch.int32:
+    dtype = mask.dtype
+    if dtype is torch.int32:
         return mask.contiguous(), _lib.MASK_I32
-    if mask.dtype in (torch.bool, torch.uint8):
+    if dtype is torch.bool or dtype is torch.uint8:
         return mask.contiguous().view(torch.uint8), _lib.MASK_U8
     active = mask > 0 if mode == _lib.MODE_PACKED_CAUSAL else mask != 0
     return active.to(torch.uint8).contiguous(), _lib.MASK_U8
@@ -114,7 +121,7 @@ class Plan:
 
     @property
     def nbytes(self) -> int:
-        return self.buf.numel()
+        return self.buf.numel()  # uint8
 
     def section(self, index: int, dtype: torch.dtype, shape: tuple[int, ...]) -> torch.Tensor:
         offs = _lib.plan_layout(self.batch, self.q_len, self.kv_len)
@@ -148,13 +155,17 @@ def block_map(segment_ids: torch.Tensor | None, mask: torch.Tensor, mode: int,
         _require_shape(segment_ids, (batch, q_len), "segment_ids")
     device = require_device(mask) if segment_ids is None else require_device(mask, segment_ids)
     m, mcode = as_mask(mask, mode)
-    seg = None if segment_ids is None else segment_ids.to(torch.int32).contiguous()
+    seg = segment_ids
+    if seg is not None:
+        if seg.dtype is not torch.int32:
+            seg = seg.to(torch.int32)
+        seg = seg.contiguous()
     nbytes = _lib.LIB.mf_plan_bytes(batch, q_len, kv_len)
     if nbytes == 0:
         raise ValueError("Sizes must be positive")
     buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    _lib.check(_lib.LIB.mf_block_map(_ptr(seg), _ptr(m), mcode, mode, batch, q_len, kv_len,
-                                     _ptr(buf), nbytes, _stream(device)))
+    _lib.check(_lib.LIB.mf_block_map(_ptr(seg), m.data_ptr(), mcode, mode, batch, q_len, kv_len,
+                                     buf.data_ptr(), nbytes, _raw_stream(device.index)))
     _BLOCK_MAP_CALLS[0] += 1
     return Plan(buf, batch, q_len, kv_len, mode)
 
@@ -186,15 +197,15 @@ def check_attention_operands(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     plan must have been built for the same batch, lengths and mode.
     """
     code = same_dtype("query, key and value", q, k, v)
-    if q.dim() != 4 or k.dim() != 4 or k.shape != v.shape or q.shape[0] != k.shape[0] \
-            or q.shape[3] != k.shape[3]:
+    qs, ks = q.shape, k.shape
+    if len(qs) != 4 or len(ks) != 4 or ks != v.shape or qs[0] != ks[0] or qs[3] != ks[3]:
         raise ValueError("Packed attention query/KV shapes are incompatible")
     require_contiguous("query, key and value", q, k, v)
     if plan is not None:
-        if (plan.batch, plan.q_len, plan.kv_len) != (q.shape[0], q.shape[1], k.shape[1]):
+        if plan.batch != qs[0] or plan.q_len != qs[1] or plan.kv_len != ks[1]:
             raise ValueError(
                 f"plan was built for batch {plan.batch}, lengths {plan.q_len}/{plan.kv_len}; "
-                f"the call has {q.shape[0]}, {q.shape[1]}/{k.shape[1]}")
+                f"the call has {qs[0]}, {qs[1]}/{ks[1]}")
         if mode is not None and plan.mode != mode:
             raise ValueError(f"plan was built for mask mode {plan.mode}, the call uses {mode}")
     return code
@@ -205,12 +216,12 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: Plan, mode
     code = check_attention_operands(q, k, v, plan, mode)
     device = require_device(q, k, v)
     b, t, hq, d = q.shape
-    s, hkv = k.shape[1], k.shape[2]
+    _, s, hkv, _ = k.shape
     out = torch.empty_like(q)
     lse = torch.empty((b, hq, t), dtype=torch.float32, device=device)
-    _lib.check(_lib.LIB.mf_attn_fwd(_ptr(q), _ptr(k), _ptr(v), code, b, t, s, hq, hkv, d, mode,
-                                    float(scale), _ptr(plan.buf), plan.nbytes, _ptr(out),
-                                    _ptr(lse), _stream(device)))
+    _lib.check(_lib.LIB.mf_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), code, b, t, s, hq,
+                                    hkv, d, mode, float(scale), plan.buf.data_ptr(), plan.nbytes,
+                                    out.data_ptr(), lse.data_ptr(), _raw_stream(device.index)))
     return out, lse
 
 
@@ -250,11 +261,12 @@ def attn_fwd_rope_q(q_raw: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 def attn_bwd(q, k, v, out, dout, lse, plan: Plan, mode: int, scale: float):
     check_attention_operands(q, k, v, plan, mode)
     code = same_dtype("query, key, value, output and its gradient", q, k, v, out, dout)
-    if out.shape != q.shape or dout.shape != q.shape:
+    qs = q.shape
+    if out.shape != qs or dout.shape != qs:
         raise ValueError("the output and its gradient must have the query's shape")
     require_contiguous("the output and its gradient", out, dout)
-    b, t, hq, d = q.shape
-    s, hkv = k.shape[1], k.shape[2]
+    b, t, hq, d = qs
+    _, s, hkv, _ = k.shape
     _require_lse(lse, b, hq, t)
     device = require_device(q, k, v, out, dout, lse)
     dq = torch.empty_like(q)
@@ -262,10 +274,11 @@ def attn_bwd(q, k, v, out, dout, lse, plan: Plan, mode: int, scale: float):
     dv = torch.empty_like(v)
     ws_bytes = _lib.LIB.mf_attn_bwd_workspace_bytes(b, t, hq)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-    _lib.check(_lib.LIB.mf_attn_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse),
-                                    code, b, t, s, hq, hkv, d, mode, float(scale), _ptr(plan.buf),
-                                    plan.nbytes, _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws), ws_bytes,
-                                    _stream(device)))
+    _lib.check(_lib.LIB.mf_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                    dout.data_ptr(), lse.data_ptr(), code, b, t, s, hq, hkv, d,
+                                    mode, float(scale), plan.buf.data_ptr(), plan.nbytes,
+                                    dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(),
+                                    ws_bytes, _raw_stream(device.index)))
     return dq, dk, dv
 
 
@@ -323,13 +336,14 @@ def attn_bwd_dkdv(q, k, v, dout, lse, plan: Plan, mode: int, scale: float, ws, d
 
 
 def _check_decode_shapes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
-    if (q.dim() != 4 or q.shape[1] != 1 or k_cache.dim() != 4 or k_cache.shape != v_cache.shape
-            or k_cache.shape[0] != q.shape[0] or k_cache.shape[3] != q.shape[3]):
+    qs, ks = q.shape, k_cache.shape
+    if (len(qs) != 4 or qs[1] != 1 or len(ks) != 4 or ks != v_cache.shape or ks[0] != qs[0]
+            or ks[3] != qs[3]):
         raise ValueError("Cached attention query/KV shapes are incompatible")
 
 
 def _check_lengths(lengths: torch.Tensor, batch: int, what: str) -> None:
-    if lengths.dtype != torch.int32 or tuple(lengths.shape) != (batch,) \
+    if lengths.dtype is not torch.int32 or lengths.shape != (batch,) \
             or not lengths.is_contiguous():
         raise ValueError(f"{what} must be a contiguous int32 [{batch}] tensor")
 
@@ -341,7 +355,7 @@ def decode_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor,
     code = same_dtype("query, new key/value and the KV caches", q, k_new, v_new, k_cache, v_cache)
     _check_decode_shapes(q, k_cache, v_cache)
     b, _, hq, d = q.shape
-    cap, hkv = k_cache.shape[1], k_cache.shape[2]
+    _, cap, hkv, _ = k_cache.shape
     for t in (k_new, v_new):
         _require_shape(t, (b, 1, hkv, d), "the new key/value rows")
     _check_lengths(positions, b, "positions")
@@ -365,7 +379,7 @@ def decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     code = same_dtype("query and the KV caches", q, k_cache, v_cache)
     _check_decode_shapes(q, k_cache, v_cache)
     b, _, hq, d = q.shape
-    cap, hkv = k_cache.shape[1], k_cache.shape[2]
+    _, cap, hkv, _ = k_cache.shape
     _check_lengths(lengths, b, "lengths")
     device = require_device(q, k_cache, v_cache, lengths)
     q, k_cache, v_cache = q.contiguous(), k_cache.contiguous(), v_cache.contiguous()
