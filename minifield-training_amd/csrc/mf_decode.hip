@@ -539,10 +539,9 @@ __global__ __launch_bounds__(512) void decode_bf16_kernel(DecArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// bf16 decode over whole token rows: one wave per (row, 128-token chunk)
-// item covering every KV head.  A token's K (or V) row -- Hkv heads x 128 B,
-// contiguous in the [B, cap, Hkv, 64] cache -- is read by 8 * Hkv lanes with
-// one non-temporal 16-byte load each, so a wave streams the chunk's rows as
+// bf16 decode over whole token rows: a token's K (or V) row -- Hkv heads x 128
+// B, contiguous in the [B, cap, Hkv, 64] cache -- is read by 8 * Hkv lanes with
+// one 16-byte load each (non-temporal for caches that stream), so a wave streams its tokens' rows as
 // one contiguous range (the access pattern that reaches the HBM read
 // ceiling on this part, where one wave per (row, chunk, head) reads 8
 // separate 128-byte pieces per instruction).  Lane = (token j of the TPL =
@@ -552,8 +551,16 @@ __global__ __launch_bounds__(512) void decode_bf16_kernel(DecArgs a) {
 // the group holds the same score; the online softmax state (max, sum) and
 // the P V accumulator of its 8 dims live in the lane.  8 tokens of K and V
 // are in flight per lane (16 loads).  Lanes of different j merge their
-// states at the end (log-sum-exp), and the (max, sum, acc) of the chunk go
-// to the partial buffer the combine kernel reads.
+// states at the end (log-sum-exp), the block's waves merge through LDS, and
+// the block's (max, sum, acc) go to the partial buffer the combine kernel
+// reads (or, when the cache is one block long, its output to `out`).
+//
+// Items are 128 tokens of a row; W waves share one.  W = 1: four items a
+// workgroup, numbered by a scan of the lengths so that the grid's first waves
+// are the ones with work: for calls with enough items to keep HBM busy.  Fewer
+// items are bound by how long one takes, so a workgroup takes one item with
+// several waves, merged through LDS: as many as can have one round of loads
+// each (16 / TPL), or four.  launch_decode has the rule and what each measures.
 // ---------------------------------------------------------------------------
 constexpr int kRowChunk = 128;  // tokens per work item of the row kernel
 constexpr int kRowUnroll = 8;   // tokens per lane in flight (K and V)
@@ -590,37 +597,57 @@ __device__ __forceinline__ int row_chunks_c(const DecArgs& a, int base, int chun
   return r < a.B ? (eff_len(raw_length(a.lengths, a.positions, r), a.cap) + chunk - 1) / chunk : 0;
 }
 
+// Waves of an item that is to finish soonest: one round of loads (8 TPL tokens)
+// each.  (Sixteen waves leave 128 registers each, which five heads and more
+// exceed: fewer waves take several rounds there.)
 template <int G, int TPL>
-__global__ __launch_bounds__(256) void decode_rows_kernel(DecArgs a) {
+constexpr int rows_most_waves() {
+  return G == 8 ? (TPL < 8 ? 4 : 2) : TPL == 1 && G > 4 ? 8 : 16 / TPL;
+}
+
+template <int G, int TPL, int W, bool KEEP_V = true>
+__global__ __launch_bounds__((W == 1 ? 256 : 64 * W)) void decode_rows_kernel(DecArgs a) {
+  constexpr bool BLOCK = W > 1;
   constexpr int kHkv = 8 / TPL;
+  constexpr int kWaveTok = kRowChunk / W;
   const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
   const int j = lane / (8 * kHkv);           // token of a load
   const int h = (lane >> 3) % kHkv;          // KV head
   const int dl = lane & 7;                   // 8-dim slice
-  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
-  // (row, chunk) of this item: rows' chunk counts scanned 64 rows at a time
-  int b = -1, chunk = 0;
-  for (int base = 0, carry = 0; base < a.B; base += 64) {
-    const int incl = wave_prefix(row_chunks_c(a, base, kRowChunk));
-    const int tot = __shfl(incl, 63);
-    if (item < carry + tot) {
-      const int k = __popcll(__ballot(carry + incl <= item));
-      b = base + k;
-      chunk = item - carry - (k > 0 ? __shfl(incl, k - 1) : 0);
-      break;
+  int b, chunk;
+  if constexpr (!BLOCK) {
+    // (row, chunk) of this wave: rows' chunk counts scanned 64 rows at a time
+    const int item = blockIdx.x * 4 + wave;
+    b = -1;
+    chunk = 0;
+    for (int base = 0, carry = 0; base < a.B; base += 64) {
+      const int incl = wave_prefix(row_chunks_c(a, base, kRowChunk));
+      const int tot = __shfl(incl, 63);
+      if (item < carry + tot) {
+        const int k = __popcll(__ballot(carry + incl <= item));
+        b = base + k;
+        chunk = item - carry - (k > 0 ? __shfl(incl, k - 1) : 0);
+        break;
+      }
+      carry += tot;
     }
-    carry += tot;
+    b = uniform(b);
+    if (b < 0) return;  // past the last item (the grid is sized for full rows)
+    chunk = uniform(chunk);
+  } else {
+    b = blockIdx.x / a.maxc;
+    chunk = blockIdx.x - b * a.maxc;
   }
-  b = uniform(b);
-  if (b < 0) return;  // past the last item (the grid is sized for full rows)
-  chunk = uniform(chunk);
   const float c = a.scale_log2;
   const float tau2 = 8.f;  // lazy rescale threshold, log2 units
   const int raw = uniform(raw_length(a.lengths, a.positions, b));
   const bool flat = raw <= 0;  // every slot masked: uniform weights
   const int len = eff_len(raw, a.cap);
-  const int t0 = chunk * kRowChunk;
-  const int last = t0 + min(kRowChunk, len - t0) - 1;
+  if (BLOCK && chunk * kRowChunk >= len) return;  // (the whole workgroup)
+  // the wave's tokens t0 .. last; none when last < t0
+  const int t0 = chunk * kRowChunk + (BLOCK ? wave * kWaveTok : 0);
+  const int last = min(t0 + kWaveTok, len) - 1;
   const int slot = a.positions ? uniform(min(max(a.positions[b], 0), a.cap - 1)) : -1;
   const size_t row_elems = (size_t)kHkv * kD;  // one token's row
   const bf16* kbase = reinterpret_cast<const bf16*>(a.k) + (size_t)b * a.cap * row_elems;
@@ -646,16 +673,16 @@ __global__ __launch_bounds__(256) void decode_rows_kernel(DecArgs a) {
   constexpr int kStep = TPL * kRowUnroll;  // tokens per iteration over the wave
   for (int tb = t0; tb <= last; tb += kStep) {
     u32x4 kr[kRowUnroll], vr[kRowUnroll];
+    // (addresses selected, not loads: a branch per token would keep the loads
+    // of an iteration from being issued back to back)
 #pragma unroll
     for (int u = 0; u < kRowUnroll; ++u) {
       const int t = min(tb + j + TPL * u, last);
-      if (t == slot) {
-        kr[u] = ld_u32x4(knew);
-        vr[u] = ld_u32x4(vnew);
-      } else {
-        kr[u] = ld_nt(kbase + (size_t)t * row_elems + lane_off);
-        vr[u] = ld_nt(vbase + (size_t)t * row_elems + lane_off);
-      }
+      const size_t off = (size_t)t * row_elems + lane_off;
+      const bf16* kp = t == slot ? knew : kbase + off;
+      const bf16* vp = t == slot ? vnew : vbase + off;
+      kr[u] = BLOCK ? ld_u32x4(kp) : ld_nt(kp);
+      vr[u] = KEEP_V ? ld_u32x4(vp) : ld_nt(vp);
     }
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -711,17 +738,73 @@ __global__ __launch_bounds__(256) void decode_rows_kernel(DecArgs a) {
   if constexpr (TPL >= 2) merge_lanes<G>(m2, l, acc, 32);
   if constexpr (TPL >= 4) merge_lanes<G>(m2, l, acc, 16);
   if constexpr (TPL >= 8) merge_lanes<G>(m2, l, acc, 8);
-  if (j != 0) return;
+  if constexpr (!BLOCK) {
+    if (j != 0) return;
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float* dst = a.partial + (((size_t)b * a.Hq + h * G + g) * a.maxc + chunk) * (2 + kD);
-    f32x4 lo = {acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
-    f32x4 hi = {acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
-    *reinterpret_cast<f32x4*>(dst + 2 + 8 * dl) = lo;
-    *reinterpret_cast<f32x4*>(dst + 2 + 8 * dl + 4) = hi;
-    if (dl == 0) {
-      dst[0] = m2[g];
-      dst[1] = l[g];
+    for (int g = 0; g < G; ++g) {
+      float* dst = a.partial + (((size_t)b * a.Hq + h * G + g) * a.maxc + chunk) * (2 + kD);
+      f32x4 lo = {acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
+      f32x4 hi = {acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
+      *reinterpret_cast<f32x4*>(dst + 2 + 8 * dl) = lo;
+      *reinterpret_cast<f32x4*>(dst + 2 + 8 * dl + 4) = hi;
+      if (dl == 0) {
+        dst[0] = m2[g];
+        dst[1] = l[g];
+      }
+    }
+    return;
+  }
+  // the item's waves: every wave scales its state to the common max, and the
+  // scaled sums and outputs are added in wave order, GP heads at a time
+  // (lane-derived values afresh, not kept across the loop)
+  const int elane = fresh_lane_id();
+  const int eh = (elane >> 3) % kHkv;
+  constexpr int GP = W >= 16 || G == 1 ? 1 : 2;
+  constexpr int kLanes = 8 * kHkv;
+  constexpr int kPart = kLanes + 1;  // odd pitch: the dims of a lane on different banks
+  __shared__ float wm[W][GP][kLanes];
+  __shared__ float wv[W][GP][9][kPart];  // sum, then the lane's 8 output dims
+#pragma unroll
+  for (int g0 = 0; g0 < G; g0 += GP) {
+    if (elane < kLanes)
+#pragma unroll
+      for (int gi = 0; gi < GP; ++gi)
+        if (g0 + gi < G) wm[wave][gi][elane] = m2[g0 + gi];
+    __syncthreads();
+    if (elane < kLanes)
+#pragma unroll
+      for (int gi = 0; gi < GP; ++gi) {
+        if (g0 + gi >= G) continue;
+        const int g = g0 + gi;
+        float top = wm[0][gi][elane];
+#pragma unroll
+        for (int w = 1; w < W; ++w) top = fmaxf(top, wm[w][gi][elane]);
+        const float wt = m2[g] == kNegInf ? 0.f : fast_exp2(m2[g] - top);
+        wv[wave][gi][0][elane] = l[g] * wt;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wv[wave][gi][1 + i][elane] = acc[g][i] * wt;
+        if (wave == 0 && (elane & 7) == 0)
+          a.partial[(((size_t)b * a.Hq + eh * G + g) * a.maxc + chunk) * (2 + kD)] = top;
+      }
+    __syncthreads();
+    // thread = (head of the round, KV head, dim)
+    for (int e = 64 * wave + elane; e < GP * kHkv * kD; e += 64 * W) {
+      const int gi = e / (kHkv * kD), hh = e / kD % kHkv, d = e % kD;
+      if (g0 + gi >= G) break;
+      float o = 0.f, sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        o += wv[w][gi][1 + (d & 7)][hh * 8 + (d >> 3)];
+        sum += wv[w][gi][0][hh * 8];
+      }
+      const size_t row = (size_t)b * a.Hq + hh * G + g0 + gi;
+      if (a.maxc == 1) {
+        reinterpret_cast<bf16*>(a.out)[row * kD + d] = (bf16)(o / sum);
+      } else {
+        float* dst = a.partial + (row * a.maxc + chunk) * (2 + kD);
+        dst[2 + d] = o;
+        if (d == 0) dst[1] = sum;
+      }
     }
   }
 }
@@ -772,14 +855,13 @@ size_t decode_workspace_bytes(int batch, int cap, int Hq, int chunk) {
          sizeof(float) * (size_t)batch * Hq * maxc * (2 + kD);
 }
 
-// Tokens per partial of the path a call takes: the row kernel (bf16, G and
-// Hkv in {1, 2, 4, 8}), the older bf16 streaming kernel (other power-of-two
-// G), or the LDS-staged kernels (fp32, other G).
+// Tokens per partial of the path a call takes: the row kernel (bf16, G up to
+// 8, Hkv in {1, 2, 4, 8}), the older bf16 streaming kernel (power-of-two G
+// over other Hkv), or the LDS-staged kernels (fp32, other G).
 int decode_chunk(bool f32) { return f32 ? 128 : kDecChunk; }
 
 bool decode_rows_path(bool f32, int G, int Hkv) {
-  return !f32 && (G == 1 || G == 2 || G == 4 || G == 8) &&
-         (Hkv == 1 || Hkv == 2 || Hkv == 4 || Hkv == 8);
+  return !f32 && G <= kMaxG && (Hkv == 1 || Hkv == 2 || Hkv == 4 || Hkv == 8);
 }
 
 // workspace bytes that serve every path (the smallest chunk has the most
@@ -787,6 +869,25 @@ bool decode_rows_path(bool f32, int G, int Hkv) {
 size_t decode_workspace_bytes_any(int batch, int cap, int Hq) {
   return decode_workspace_bytes(batch, cap, Hq, kRowChunk < 128 ? kRowChunk : 128);
 }
+
+// Items (128 tokens of a full row, over all rows) up to which a workgroup takes
+// one: with the most waves while every CU has at most one item, with four up to
+// two items per CU.  us of decode + combine with one wave per item and a
+// branch per load (before), with four waves, with the most, and with one wave
+// (16/8 heads, ragged lengths, inputs rotating):
+//   1 x 4096     32 items    30.0   13.5   11.5
+//   8 x 4096    256          32.8   15.7   14.0
+//   8 x 8192    512          34.5   20.4   25.5
+//   64 x 1024   512          33.7   23.0   28.3
+//   16 x 8192  1024          36.4   42.1   43.9   36.6
+//   64 x 4096  2048          67.0   70.3   93.5   62.6
+//   64 x 8192  4096         112.5  117    152    111.1
+constexpr long long kMostWavesItems = 256;
+constexpr long long kFourWavesItems = 512;
+// Caches (K and V, all rows) that fit the 256 MB last-level cache keep V
+// cacheable, larger ones stream: 16 x 8192 takes 36.6 us so and 38.4 with both
+// streamed, 64 x 8192 114.0 and 111.1, 256 x 1024 69.1 and 65.3.
+constexpr long long kKeepBytes = 256ll << 20;
 
 hipError_t launch_decode(const void* q, const void* k, const void* v, const int32_t* lengths,
                          bool f32, int batch, int cap, int Hq, int Hkv, float scale, void* out,
@@ -819,7 +920,7 @@ hipError_t launch_decode(const void* q, const void* k, const void* v, const int3
                                        align256(sizeof(int) * (size_t)batch));
   // The register-streaming bf16 kernel walks the chunks and appends itself;
   // the LDS-staged kernels (fp32, other head groups) need the prep pass.
-  const bool streaming = !f32 && (a.G == 1 || a.G == 2 || a.G == 4 || a.G == 8);
+  const bool streaming = rows || (!f32 && (a.G == 1 || a.G == 2 || a.G == 4 || a.G == 8));
   if (!streaming) {
     if (f32)
       hipLaunchKernelGGL((decode_prep_kernel<4>), dim3(1), dim3(256), 0, stream, a);
@@ -838,22 +939,40 @@ hipError_t launch_decode(const void* q, const void* k, const void* v, const int3
     return hipGetLastError();
   }
   if (rows) {
-    // one wave per (row, chunk) item; the grid covers full rows, waves past
-    // the last item exit at once
-    const long long waves = (long long)batch * a.maxc;
-    const dim3 grid((unsigned)((waves + 3) / 4));
+    // the grid covers full rows; workgroups (waves) past a row's (the last)
+    // chunk exit at once
+    const long long items = (long long)batch * a.maxc;
+    const bool most = items <= kMostWavesItems;
+    const bool four = !most && items <= kFourWavesItems;
+    const bool keep_v = (long long)batch * cap * Hkv * kD * (2 * sizeof(bf16)) <= kKeepBytes;
+    const dim3 grid((unsigned)(most || four ? items : (items + 3) / 4));
     switch (a.G * 16 + Hkv) {
-#define MF_ROWS(GG, HH) \
-  case GG * 16 + HH: hipLaunchKernelGGL((decode_rows_kernel<GG, 8 / HH>), grid, dim3(256), 0, stream, a); break;
-      MF_ROWS(1, 1) MF_ROWS(1, 2) MF_ROWS(1, 4) MF_ROWS(1, 8)
-      MF_ROWS(2, 1) MF_ROWS(2, 2) MF_ROWS(2, 4) MF_ROWS(2, 8)
-      MF_ROWS(4, 1) MF_ROWS(4, 2) MF_ROWS(4, 4) MF_ROWS(4, 8)
-      MF_ROWS(8, 1) MF_ROWS(8, 2) MF_ROWS(8, 4) MF_ROWS(8, 8)
+#define MF_ROWS_W(GG, HH, WW, KEEP)                                                   \
+  hipLaunchKernelGGL((decode_rows_kernel<GG, 8 / HH, WW, KEEP>), grid,                \
+                     dim3(WW == 1 ? 256 : 64 * WW), 0, stream, a)
+#define MF_ROWS(GG, HH)                                                               \
+  case GG * 16 + HH:                                                                  \
+    if (most)                                                                         \
+      MF_ROWS_W(GG, HH, (rows_most_waves<GG, 8 / HH>()), true);                       \
+    else if (four)                                                                    \
+      MF_ROWS_W(GG, HH, (8 / HH < 8 ? 4 : 2), true);                                  \
+    else if (keep_v)                                                                  \
+      MF_ROWS_W(GG, HH, 1, true);                                                     \
+    else                                                                              \
+      MF_ROWS_W(GG, HH, 1, false);                                                    \
+    break;
+#define MF_ROWS_G(GG) MF_ROWS(GG, 1) MF_ROWS(GG, 2) MF_ROWS(GG, 4) MF_ROWS(GG, 8)
+      MF_ROWS_G(1) MF_ROWS_G(2) MF_ROWS_G(3) MF_ROWS_G(4)
+      MF_ROWS_G(5) MF_ROWS_G(6) MF_ROWS_G(7) MF_ROWS_G(8)
+#undef MF_ROWS_G
 #undef MF_ROWS
+#undef MF_ROWS_W
       default: return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL((decode_combine_kernel<false>), dim3(batch * Hq), dim3(64 * kCombineWaves),
-                       0, stream, a);
+    // (a workgroup that holds a whole row writes the output itself)
+    if (!(most || four) || a.maxc > 1)
+      hipLaunchKernelGGL((decode_combine_kernel<false>), dim3(batch * Hq),
+                         dim3(64 * kCombineWaves), 0, stream, a);
     return hipGetLastError();
   }
   // bf16: persistent grid of 4-wave blocks over (chunk item, KV head)
