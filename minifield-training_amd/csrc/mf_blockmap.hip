@@ -30,29 +30,11 @@ struct MapArgs {
   int batch, q_len, kv_len;
   PlanLayout lay;
   char* plan;
-  int ids_ready;  // qid/kid already hold the canonical ids (key-mask mode, placements)
+  int ids_ready;  // qid/kid already hold the canonical ids (placements)
 };
 
 __device__ __forceinline__ int* plan_i32(char* plan, size_t off) {
   return reinterpret_cast<int*>(plan + off);
-}
-
-// Key-mask mode ids, one block per (position chunk, row): every query of a
-// row with at least one active key gets id 1 (present = any(mask[b, :]),
-// bidirectional.py:23), key j gets id 1 iff mask != 0.  The packed modes'
-// ids are derived inside the run pass instead.
-__global__ __launch_bounds__(256) void token_ids_kernel(MapArgs a) {
-  const int b = blockIdx.y;
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  int* qid = plan_i32(a.plan, a.lay.qid) + (size_t)b * a.lay.tq_pad;
-  int* kid = plan_i32(a.plan, a.lay.kid) + (size_t)b * a.lay.tk_pad;
-  int any = 0;
-  for (int j = threadIdx.x; j < a.kv_len; j += blockDim.x)
-    any |= mask_at(a.mask, a.mask_u8, (long)b * a.kv_len + j) != 0;
-  any = __syncthreads_or(any);
-  if (p < a.lay.tq_pad) qid[p] = (p < a.q_len && any) ? 1 : 0;
-  if (p < a.lay.tk_pad)
-    kid[p] = (p < a.kv_len && mask_at(a.mask, a.mask_u8, (long)b * a.kv_len + p) != 0) ? 1 : 0;
 }
 
 // Canonical id of token p of row b in the packed modes (q_len == kv_len).
@@ -65,11 +47,29 @@ __device__ __forceinline__ int packed_id(const MapArgs& a, int b, int p) {
   return active ? s : 0;
 }
 
+// Key-mask mode: whether row b has an active key (bidirectional.py:23), for a
+// whole wave.  512 keys a round, until one is active: the first round in all
+// but rows that open with padding.
+__device__ __forceinline__ bool row_has_key(const MapArgs& a, int b) {
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < a.kv_len; base += 512) {
+    int any = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int p = min(base + 64 * i + lane, a.kv_len - 1);
+      any |= mask_at(a.mask, a.mask_u8, (long)b * a.kv_len + p);
+    }
+    if (__any(any != 0)) return true;
+  }
+  return false;
+}
+
 // One wave per (tile, row): tiles [0, nq) are query tiles, [nq, nq+nk) key
-// tiles.  Writes the ordered maximal runs of equal nonzero ids.  In the
-// packed modes it also derives the tile's canonical ids from the segment ids
-// and mask and stores them (query tiles into qid, key tiles into kid), so no
-// separate id pass runs.
+// tiles.  Writes the ordered maximal runs of equal nonzero ids.  It also
+// derives the tile's canonical ids and stores them (query tiles into qid, key
+// tiles into kid), so no separate id pass runs: in the packed modes from the
+// segment ids and mask; in the key-mask mode every query of a row with an
+// active key gets id 1, and key j iff its mask is set (bidirectional.py:22-25).
 __global__ __launch_bounds__(64) void tile_runs_kernel(MapArgs a) {
   const int b = blockIdx.y;
   const int t = blockIdx.x;
@@ -83,16 +83,22 @@ __global__ __launch_bounds__(64) void tile_runs_kernel(MapArgs a) {
               rec_bytes * ((size_t)b * (a.lay.nq + a.lay.nk) + (size_t)t);
   Run* runs = reinterpret_cast<Run*>(rec + sizeof(int));
   const int p0 = tile * kTile;
+  const bool row_has = a.mode == 2 && is_q && !a.ids_ready && row_has_key(a, b);
   int x[2];
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
     const int p = p0 + half * 64 + lane;
     if (a.ids_ready) {
       x[half] = ids[p];
-    } else {
-      x[half] = packed_id(a, b, p);
-      ids[p] = x[half];
+      continue;
     }
+    if (a.mode != 2)
+      x[half] = packed_id(a, b, p);
+    else if (is_q)
+      x[half] = p < a.q_len && row_has;
+    else
+      x[half] = p < a.kv_len && mask_at(a.mask, a.mask_u8, (long)b * a.kv_len + p) != 0;
+    ids[p] = x[half];
   }
   int n_start = 0, n_stop = 0;
 #pragma unroll
@@ -378,11 +384,71 @@ __global__ __launch_bounds__(256) void placement_ids_kernel(MapArgs a, const int
   }
 }
 
+// The same order for up to kRankItems items a side, one per thread: an item's
+// place is its bucket's start, plus the bucket's items in earlier waves, plus
+// those in earlier lanes (the lanes of a bucket from one ballot per bucket
+// bit).  2.2 us for 72 items between idle neighbours, where the counting sort
+// above, whose threads take several items and scan the buckets serially, takes
+// 3.2; behind a busy kernel a launch of this size costs 4.6 us either way.
+constexpr int kRankItems = 1024;
+
+__global__ __launch_bounds__(kRankItems) void order_rank_kernel(MapArgs a) {
+  static_assert(kOrderBuckets == 64, "a lane per bucket");
+  __shared__ int hist[kRankItems / 64][kOrderBuckets];  // then: the bucket's items in earlier waves
+  __shared__ int start[kOrderBuckets];
+  const bool qside = blockIdx.x == 0;
+  const int n = a.batch * (qside ? a.lay.nq : a.lay.nk);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const bool live = t < n;
+  const int bucket = live ? order_bucket(plan_i32(a.plan, qside ? a.lay.qcnt : a.lay.kcnt)[t]) : 0;
+  uint64_t same = __ballot(live);
+#pragma unroll
+  for (int bit = 0; bit < 6; ++bit) {
+    const bool set = (bucket >> bit) & 1;
+    const uint64_t m = __ballot(set);
+    same &= set ? m : ~m;
+  }
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const int before = __popcll(same & below);
+  hist[wave][lane] = 0;
+  if (live && before == 0) hist[wave][bucket] = __popcll(same);
+  __syncthreads();
+  if (wave == 0) {
+    int total = 0;
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) {
+      const int c = hist[w][lane];
+      hist[w][lane] = total;
+      total += c;
+    }
+    int incl = total;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int y = __shfl_up(incl, off);
+      if (lane >= off) incl += y;
+    }
+    start[lane] = incl - total;
+  }
+  __syncthreads();
+  if (live)
+    plan_i32(a.plan, qside ? a.lay.qorder : a.lay.korder)[start[bucket] + hist[wave][bucket] + before] = t;
+}
+
+// Three launches.  Each costs about 4.7 us behind a busy kernel, whatever it
+// does, so the key-mask mode derives its ids in the run pass too instead of in
+// a launch of its own (forward of 24 x 333 padded rows: 35.5 -> 31.8 us with
+// the shorter order).  One workgroup for the whole map measured worse beyond a
+// few tiles (24 x 333: 21 us against 13.6, 1 x 5003: 25.6 against 14.3: the run
+// extraction is ~250 instructions per tile and one CU issues all of it).
 static void launch_map_tail(const MapArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL(tile_runs_kernel, dim3(a.lay.nq + a.lay.nk, a.batch), dim3(64), 0, stream, a);
   hipLaunchKernelGGL(tile_lists_kernel, dim3(a.lay.nq + a.lay.nk, a.batch),
                      dim3(list_threads(a.lay.nq, a.lay.nk)), 0, stream, a);
-  hipLaunchKernelGGL(order_kernel, dim3(2), dim3(kOrderThreads), 0, stream, a);
+  const long long items = (long long)a.batch * (a.lay.nq > a.lay.nk ? a.lay.nq : a.lay.nk);
+  if (items <= kRankItems)
+    hipLaunchKernelGGL(order_rank_kernel, dim3(2), dim3((unsigned)((items + 63) / 64 * 64)), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL(order_kernel, dim3(2), dim3(kOrderThreads), 0, stream, a);
 }
 
 hipError_t launch_block_map_placements(const int32_t* placements, int count, int mode, int batch,
@@ -421,13 +487,7 @@ hipError_t launch_block_map(const int32_t* seg, const void* mask, int mask_u8, i
   a.kv_len = kv_len;
   a.lay = plan_layout(batch, q_len, kv_len);
   a.plan = reinterpret_cast<char*>(plan);
-  // packed modes: the run pass derives the ids itself; the key-mask mode
-  // needs a row-wide "any key active" first
-  a.ids_ready = mode == 2;
-  if (a.ids_ready) {
-    const int pad = a.lay.tq_pad > a.lay.tk_pad ? a.lay.tq_pad : a.lay.tk_pad;
-    hipLaunchKernelGGL(token_ids_kernel, dim3((pad + 255) / 256, batch), dim3(256), 0, stream, a);
-  }
+  a.ids_ready = 0;
   launch_map_tail(a, stream);
   return hipGetLastError();
 }
