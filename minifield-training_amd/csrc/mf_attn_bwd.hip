@@ -664,15 +664,8 @@ void bwd_dq_bf16_kernel(BwdArgs a) {
     a.ndelta[lj] = -dlt;
     a.lse2[lj] = lse2;
   }
-#pragma unroll
-  for (int db = 0; db < 2; ++db)
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int d0 = db * 32 + 8 * g4 + 4 * ehalf;
-      const bf16x4 o = scaled_bf16x4(dqacc[db], g4 * 4, a.scale, qactive);
-      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.dq) +
-                                 (((size_t)b * a.T + eqpos) * a.Hq + head) * kD + d0) = o;
-    }
+  store_bf16_rows(reinterpret_cast<bf16*>(a.dq) + (((size_t)b * a.T + eqpos) * a.Hq + head) * kD,
+                  dqacc, a.scale, qactive, ehalf);
 }
 
 // ---------------------------------------------------------------------------
@@ -718,7 +711,6 @@ void bwd_dkdv_bf16_kernel(BwdArgs a) {
   const int kt = uniform(item - b * a.nk);
   const int kpos = kt * kTile + (wave & 3) * 32 + (lane & 31);
   const int mykid = a.kid[(size_t)b * a.tk_pad + kpos];
-  const bool kvalid = kpos < a.S;
 
   bf16x8 kf[4], vf[4];
   {
@@ -927,19 +919,20 @@ void bwd_dkdv_bf16_kernel(BwdArgs a) {
   }
   wait_vmcnt<0>();
 
-  if (!kvalid) return;
+  // the lane's row and half from a fresh lane id, as in dq, and its row offset
+  // apart from the wave's scalar one (a 64-bit offset per lane spilled three
+  // registers across the loop)
+  const int elane = fresh_lane_id();
   const bool kactive = mykid != 0;
-#pragma unroll
-  for (int db = 0; db < 2; ++db)
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int d0 = db * 32 + 8 * g4 + 4 * half;
-      const size_t off = (((size_t)b * a.S + kpos) * a.Hkv + kvh) * kD + d0;
-      const bf16x4 ok = scaled_bf16x4(dkacc[db], g4 * 4, a.scale, kactive);
-      const bf16x4 ov = scaled_bf16x4(dvacc[db], g4 * 4, 1.f, kactive);
-      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.dk) + off) = ok;
-      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.dv) + off) = ov;
-    }
+  const int krow = kt * kTile + (wave & 3) * 32;
+  if ((elane & 31) < a.S - krow) {
+    const size_t off = (((size_t)b * a.S + krow) * a.Hkv + kvh) * kD;
+    const uint32_t lane_off = (elane & 31) * a.Hkv * kD;
+    store_bf16_rows(reinterpret_cast<bf16*>(a.dk) + off + lane_off, dkacc, a.scale, kactive,
+                    elane >> 5);
+    store_bf16_rows(reinterpret_cast<bf16*>(a.dv) + off + lane_off, dvacc, 1.f, kactive,
+                    elane >> 5);
+  }
 }
 
 hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const void* out,

@@ -553,15 +553,9 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
     // natural-log LSE: shift / log2(e) + ln(l)
     if (ehalf == 0)
       a.lse[((size_t)b * a.Hq + head) * a.T + eqpos] = has ? fmaf(shift, kLn2, __logf(lt)) : kPosInf;
-#pragma unroll
-    for (int db = 0; db < 2; ++db)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int d0 = db * 32 + 8 * g4 + 4 * ehalf;
-        const bf16x4 o = scaled_bf16x4(oacc[db], g4 * 4, inv, has);
-        *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.out) +
-                                   (((size_t)b * a.T + eqpos) * a.Hq + head) * kD + d0) = o;
-      }
+    store_bf16_rows(reinterpret_cast<bf16*>(a.out) +
+                        (((size_t)b * a.T + eqpos) * a.Hq + head) * kD,
+                    oacc, inv, has, ehalf);
   }
 }
 

@@ -127,6 +127,38 @@ __device__ __forceinline__ bf16x4 scaled_bf16x4(const f32x16& v, int base, float
   return __builtin_bit_cast(bf16x4, w);
 }
 
+// Writes a wave's transposed 32 x 64 accumulator tile (lane = row `lane & 31`,
+// acc[db][4 g + i] = dim 32 db + 8 g + 4 half + i) as bf16 rows `stride`
+// elements apart, scaled or zeroed as scaled_bf16x4; `row` is the lane's own
+// row.  All 64 lanes of a written row pair (l, l ^ 32) take part.
+//
+// What bounds the store is the number of L2 write requests, not the bytes: as
+// accumulated, a lane holds four neighbouring dims, and an 8-byte store per
+// four is 32 partial writes of 16 bytes.  Exchanging one group of four with the
+// other half (group g of the upper lanes against group g + 1 of the lower) gives
+// each lane eight neighbouring dims: 16-byte stores, half as many, that fill
+// whole 32-byte sectors.  us per kernel, forward / dq / dk/dv, median over the
+// three training steps below: 108 / 133 / 160 -> 104 / 129 / 154; whole step:
+// 8 x 4096 bidirectional 560 -> 546, 4 x 8192 causal 414 -> 401, 1 x 32768 of
+// short segments 236.5 -> 219.  A second exchange over 16 lanes (64 bytes of a
+// row per store) measured 216, 401 and 549: no gain outside short segments.
+__device__ __forceinline__ void store_bf16_rows(bf16* row, const f32x16 (&acc)[2], float mul,
+                                                bool keep, int half) {
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+      const u32x2 x = __builtin_bit_cast(u32x2, scaled_bf16x4(acc[db], 4 * g, mul, keep));
+      const u32x2 y = __builtin_bit_cast(u32x2, scaled_bf16x4(acc[db], 4 * g + 4, mul, keep));
+      // [0]: x of the lower lanes, y of the lower lanes (in the upper ones);
+      // [1]: x of the upper lanes (in the lower ones), y of the upper lanes
+      const auto a = __builtin_amdgcn_permlane32_swap(x[0], y[0], false, false);
+      const auto b = __builtin_amdgcn_permlane32_swap(x[1], y[1], false, false);
+      const u32x4 w = {a[0], b[0], a[1], b[1]};
+      *reinterpret_cast<u32x4*>(row + 32 * db + 8 * (g + half)) = w;
+    }
+}
+
 __device__ __forceinline__ bf16x8 ld_bf16x8(const void* p) {
   return *reinterpret_cast<const bf16x8*>(p);
 }
