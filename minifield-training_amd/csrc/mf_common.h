@@ -167,6 +167,16 @@ __device__ __forceinline__ u32x4 ld_u32x4(const void* p) {
   return *reinterpret_cast<const u32x4*>(p);
 }
 
+// Accesses to data that one pass streams through once (no reuse in L2).
+template <typename V>
+__device__ __forceinline__ V ld_stream(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+}
+template <typename V>
+__device__ __forceinline__ void st_stream(void* p, const V& v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
+}
+
 __device__ __forceinline__ void st_u32x4(void* p, const u32x4& v) {
   *reinterpret_cast<u32x4*>(p) = v;
 }

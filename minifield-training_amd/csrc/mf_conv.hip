@@ -37,14 +37,19 @@ struct ConvArgs {
 constexpr int kConvTile = 32;  // output tokens per thread
 
 // 8 elements of one token row as loaded: raw tensor words, converted when used.
-template <typename T>
+// STREAM: read as a stream (bf16 only: fp32 touches a line with two loads of
+// 16 bytes per lane, and streamed it is slower, 46 -> 52 us forward and
+// 102 -> 127 backward at 4 x 4096 tokens of 768 channels, K = 4).  The forward,
+// which re-reads K - 1 rows in kConvTile, takes 55.7 -> 48.5 us at 8 x 4096 x
+// 1024 bf16 (50.9 -> 48.1 on another card).
+template <typename T, bool STREAM>
 struct Raw8 {
   bf16x8 v;
-  __device__ __forceinline__ void load(const T* p) { v = ld_bf16x8(p); }
+  __device__ __forceinline__ void load(const T* p) { v = STREAM ? ld_stream<bf16x8>(p) : ld_bf16x8(p); }
   __device__ __forceinline__ float operator[](int e) const { return (float)v[e]; }
 };
-template <>
-struct Raw8<float> {
+template <bool STREAM>
+struct Raw8<float, STREAM> {
   f32x4 lo, hi;
   __device__ __forceinline__ void load(const float* p) {
     lo = *reinterpret_cast<const f32x4*>(p);
@@ -109,7 +114,7 @@ __global__ __launch_bounds__(256) void segmented_conv_kernel(ConvArgs a) {
   const T* cp = reinterpret_cast<const T*>(a.c);
   // ring slot k: input u's v, b and segment id, and the c gate of output
   // u - (K - 1); tokens outside the row read token 0 or T - 1 and get id 0
-  Raw8<T> vin[kAhead], bin[kAhead], cin[kAhead];
+  Raw8<T, true> vin[kAhead], bin[kAhead], cin[kAhead];
   int sin_[kAhead];
   auto issue = [&](int u, int k) {
     const int s = t0 + lo + u;
@@ -202,8 +207,10 @@ __global__ __launch_bounds__(256) void segmented_conv_kernel(ConvArgs a) {
           x0[e] = a.c ? cu[e] * acc[e] : acc[e];
           x1[e] = a.c ? cu[4 + e] * acc[4 + e] : acc[4 + e];
         }
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + off) = x0;
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + off + 4) = x1;
+        // as streams: 46.1 -> 43.2 us at 4 x 4096 x 768 (the bf16 stores gain
+        // nothing: 50.9 and 51.9 at 8 x 4096 x 1024)
+        st_stream(reinterpret_cast<float*>(a.out) + off, x0);
+        st_stream(reinterpret_cast<float*>(a.out) + off + 4, x1);
       }
     }
   }
@@ -252,38 +259,43 @@ constexpr int conv_bwd_channels() {
 }
 
 // CW elements of one token row of the backward as loaded.
-template <typename T, int CW>
-struct RawC : Raw8<T> {};
-template <>
-struct RawC<bf16, 4> {
+template <typename T, int CW, bool STREAM>
+struct RawC : Raw8<T, STREAM> {};
+template <bool STREAM>
+struct RawC<bf16, 4, STREAM> {
   bf16x4 v;
   __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const bf16x4*>(p); }
   __device__ __forceinline__ float operator[](int e) const { return (float)v[e]; }
 };
-template <>
-struct RawC<float, 4> {
+template <bool STREAM>
+struct RawC<float, 4, STREAM> {
   f32x4 v;
   __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const f32x4*>(p); }
   __device__ __forceinline__ float operator[](int e) const { return v[e]; }
 };
 
+// The backward's gradients go out as streams (nothing of the call reads them
+// again): forward and backward of 4 x 4096 x 768 fp32, K = 4, 152 -> 147.4 us,
+// 8 x 4096 x 1024 bf16, K = 4, 232 -> 228.  A consumer that reads all of them
+// right away finds less of them cached: 64 x 512 x 512 with such a pass
+// 148.3 -> 150.3, 8 x 4096 x 1024 259 -> 257, streamed loads included.
 template <typename T, int CW>
 __device__ __forceinline__ void store_row(T* p, const float (&x)[CW]) {
   if constexpr (std::is_same<T, float>::value) {
 #pragma unroll
     for (int h = 0; h < CW; h += 4) {
       const f32x4 v = {x[h], x[h + 1], x[h + 2], x[h + 3]};
-      *reinterpret_cast<f32x4*>(p + h) = v;
+      st_stream(p + h, v);
     }
   } else if constexpr (CW == 8) {
     uint32_t words[4];
 #pragma unroll
     for (int e = 0; e < 8; e += 2) words[e / 2] = pack_pair(x[e], x[e + 1]);
     const u32x4 v = {words[0], words[1], words[2], words[3]};
-    *reinterpret_cast<u32x4*>(p) = v;
+    st_stream(p, v);
   } else {
     const u32x2 v = {pack_pair(x[0], x[1]), pack_pair(x[2], x[3])};
-    *reinterpret_cast<u32x2*>(p) = v;
+    st_stream(p, v);
   }
 }
 
@@ -308,7 +320,13 @@ __device__ __forceinline__ void conv_bwd_tile(const ConvBwdArgs& a, size_t row, 
   const T* bp = reinterpret_cast<const T*>(a.b);
   const T* cp = reinterpret_cast<const T*>(a.c);
   const T* gp = reinterpret_cast<const T*>(a.g);
-  RawC<T, CW> rv[R], rb[R], rg[R], rc[R];
+  // A tile re-reads W - 1 of its neighbour's rows.  Up to W = 5 its loads still
+  // gain as streams, at W = 7 no longer.  us, forward and backward, without
+  // and with (stores as streams on both sides): 8 x 4096 x 1024 bf16, W = 3
+  // 175 -> 168, W = 5 180.7 -> 176.5; 8 x 4096 x 768, W = 5 161.5 -> 156;
+  // 9 x 1777 x 768, W = 7 119.5 -> 122
+  constexpr bool kStream = W <= 5;
+  RawC<T, CW, kStream> rv[R], rb[R], rg[R], rc[R];
   int sg[R];
   auto issue = [&](int q, int slot) {
     const int s = t0 + SMIN + q;
