@@ -56,6 +56,12 @@ template <bool F32> struct RopeRow;
 template <> struct RopeRow<false> { bf16x8 v; };
 template <> struct RopeRow<true> { f32x4 a, b; };
 
+// bf16 rows are read, and the backward's written, as streams: every row is
+// touched once, whole 128-byte lines per instruction.  24 x 4096 tokens of
+// 16/8 heads, forward and backward: 291 -> 279 us; the forward alone at
+// 8 x 4096: 39 -> 36.  fp32 keeps plain accesses (a line is touched by two
+// loads of 16 bytes per lane; streamed, the backward takes 70 us against 63),
+// and the forward keeps plain stores (36.4 us both ways).
 template <bool F32>
 __device__ __forceinline__ RopeRow<F32> load_rope_row(const void* src, size_t base) {
   RopeRow<F32> r;
@@ -64,7 +70,7 @@ __device__ __forceinline__ RopeRow<F32> load_rope_row(const void* src, size_t ba
     r.a = *reinterpret_cast<const f32x4*>(p);
     r.b = *reinterpret_cast<const f32x4*>(p + 4);
   } else {
-    r.v = ld_bf16x8(reinterpret_cast<const bf16*>(src) + base);
+    r.v = ld_stream<bf16x8>(reinterpret_cast<const bf16*>(src) + base);
   }
   return r;
 }
@@ -324,7 +330,7 @@ __device__ __forceinline__ void norm_rope_bwd_store(const RopeRow<F32>& xin,
     bf16x8 o;
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = (bf16)(inv * fmaf(-y[i], mean, dy[i]));
-    *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(dst) + base) = o;
+    st_stream(reinterpret_cast<bf16*>(dst) + base, o);
   }
 }
 
