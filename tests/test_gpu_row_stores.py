@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from _helpers import check_bf16, operands, torch_reference
+from mfattn import ops
 from mfattn.kernels import attention, bidirectional
 
 pytestmark = pytest.mark.gpu
@@ -34,3 +35,39 @@ def test_ragged_row_tiles(t, heads, device):
         for name, a, r in zip(("out", "dq", "dk", "dv"), (out.detach(), *grads), ref):
             check_bf16(f"{name} mode {mode} t {t} heads {heads}", a, r)
             assert not a[tm == 0].any(), name
+
+
+def test_outputs_at_an_eight_byte_offset(device):
+    """The 16-byte row stores into caller's buffers that start eight bytes past a 16-byte
+    boundary: the bits of the aligned call, and nothing around them touched."""
+    rng = np.random.default_rng(77)
+    q, k, v, do = operands(rng, 2, 161, 4, 2, 64, torch.bfloat16, 1.0)
+    seg = torch.ones((2, 161), dtype=torch.int32, device=device)
+    plan = ops.block_map(seg, seg, 0, 161, 161)
+    out, lse = ops.attn_fwd(q, k, v, plan, 0, 0.125)
+    ws = ops.bwd_workspace(q)
+    ops.attn_bwd_delta(out, do, lse, ws)
+
+    def buffers(n):
+        whole = torch.full((q.numel() + 16,), 7.0, dtype=torch.bfloat16, device=device)
+        return whole, [whole[at:at + n] for at in (8, 4)]
+
+    whole, views = buffers(q.numel())
+    results = []
+    for x in views:
+        whole.fill_(7.0)
+        ops.attn_bwd_dq(q, k, v, do, lse, plan, 0, 0.125, ws, x.view_as(q))
+        results.append(x.clone())
+        at = x.storage_offset()
+        assert (whole[:at] == 7).all() and (whole[at + q.numel():] == 7).all()
+    assert torch.equal(*results)
+    whole, views = buffers(k.numel())
+    results = []
+    for x in views:
+        whole.fill_(7.0)
+        dv = torch.empty_like(v)
+        ops.attn_bwd_dkdv(q, k, v, do, lse, plan, 0, 0.125, ws, x.view_as(k), dv)
+        results.append(x.clone())
+        at = x.storage_offset()
+        assert (whole[:at] == 7).all() and (whole[at + k.numel():] == 7).all()
+    assert torch.equal(*results)
