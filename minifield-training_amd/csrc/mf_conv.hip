@@ -40,7 +40,7 @@ constexpr int kConvTile = 32;  // output tokens per thread
 // STREAM: read as a stream (bf16 only: fp32 touches a line with two loads of
 // 16 bytes per lane, and streamed it is slower, 46 -> 52 us forward and
 // 102 -> 127 backward at 4 x 4096 tokens of 768 channels, K = 4).  The forward,
-// which re-reads K - 1 rows in kConvTile, takes 55.7 -> 48.5 us at 8 x 4096 x
+// which re-reads K - 1 rows in kConvTile, streams from kStreamBytes on and takes 55.7 -> 48.5 us at 8 x 4096 x
 // 1024 bf16 (50.9 -> 48.1 on another card).
 template <typename T, bool STREAM>
 struct Raw8 {
@@ -81,7 +81,7 @@ constexpr int conv_gcd(int x, int y) { return y ? conv_gcd(y, x % y) : x; }
 // K gated inputs and stored.  For bf16, the rounded tap products of a pair of
 // taps are packed by one conversion and added to the fp32 sum by one dot
 // product with (1, 1).
-template <typename T, int K>
+template <typename T, int K, bool STREAM>
 __global__ __launch_bounds__(256) void segmented_conv_kernel(ConvArgs a) {
   // input tokens whose v, b and c loads are in flight ahead of the one in use
   // (fewer for fp32, whose rows are twice as wide), chosen so that
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void segmented_conv_kernel(ConvArgs a) {
   const T* cp = reinterpret_cast<const T*>(a.c);
   // ring slot k: input u's v, b and segment id, and the c gate of output
   // u - (K - 1); tokens outside the row read token 0 or T - 1 and get id 0
-  Raw8<T, true> vin[kAhead], bin[kAhead], cin[kAhead];
+  Raw8<T, STREAM> vin[kAhead], bin[kAhead], cin[kAhead];
   int sin_[kAhead];
   auto issue = [&](int u, int k) {
     const int s = t0 + lo + u;
@@ -561,15 +561,26 @@ template <typename T>
 hipError_t launch_conv_t(const ConvArgs& a, int K, hipStream_t stream) {
   const long long threads = (long long)a.B * ((a.T + kConvTile - 1) / kConvTile) * (a.C / 8);
   const dim3 grid((unsigned)((threads + 255) / 256));
+  const size_t tensors = 2 + (a.b != nullptr) + (a.c != nullptr);
+  const bool big = (size_t)a.B * a.T * a.C * sizeof(T) * tensors >= kStreamBytes;
+  constexpr bool kBf16 = !std::is_same<T, float>::value;
   switch (K) {
-    case 1: hipLaunchKernelGGL((segmented_conv_kernel<T, 1>), grid, dim3(256), 0, stream, a); break;
-    case 2: hipLaunchKernelGGL((segmented_conv_kernel<T, 2>), grid, dim3(256), 0, stream, a); break;
-    case 3: hipLaunchKernelGGL((segmented_conv_kernel<T, 3>), grid, dim3(256), 0, stream, a); break;
-    case 4: hipLaunchKernelGGL((segmented_conv_kernel<T, 4>), grid, dim3(256), 0, stream, a); break;
-    case 5: hipLaunchKernelGGL((segmented_conv_kernel<T, 5>), grid, dim3(256), 0, stream, a); break;
-    case 6: hipLaunchKernelGGL((segmented_conv_kernel<T, 6>), grid, dim3(256), 0, stream, a); break;
-    case 7: hipLaunchKernelGGL((segmented_conv_kernel<T, 7>), grid, dim3(256), 0, stream, a); break;
-    case 8: hipLaunchKernelGGL((segmented_conv_kernel<T, 8>), grid, dim3(256), 0, stream, a); break;
+#define MF_CONV_CASE(KK)                                                                          \
+    case KK:                                                                                      \
+      if (kBf16 && big)                                                                           \
+        hipLaunchKernelGGL((segmented_conv_kernel<T, KK, kBf16>), grid, dim3(256), 0, stream, a); \
+      else                                                                                        \
+        hipLaunchKernelGGL((segmented_conv_kernel<T, KK, false>), grid, dim3(256), 0, stream, a); \
+      break;
+    MF_CONV_CASE(1)
+    MF_CONV_CASE(2)
+    MF_CONV_CASE(3)
+    MF_CONV_CASE(4)
+    MF_CONV_CASE(5)
+    MF_CONV_CASE(6)
+    MF_CONV_CASE(7)
+    MF_CONV_CASE(8)
+#undef MF_CONV_CASE
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -56,13 +56,13 @@ template <bool F32> struct RopeRow;
 template <> struct RopeRow<false> { bf16x8 v; };
 template <> struct RopeRow<true> { f32x4 a, b; };
 
-// bf16 rows are read, and the backward's written, as streams: every row is
-// touched once, whole 128-byte lines per instruction.  24 x 4096 tokens of
+// STREAM: bf16 rows are read (the backward's also written) as streams, in the
+// forward from kStreamBytes on: every row is touched once, whole 128-byte lines per instruction.  24 x 4096 tokens of
 // 16/8 heads, forward and backward: 291 -> 279 us; the forward alone at
 // 8 x 4096: 39 -> 36.  fp32 keeps plain accesses (a line is touched by two
 // loads of 16 bytes per lane; streamed, the backward takes 70 us against 63),
 // and the forward keeps plain stores (36.4 us both ways).
-template <bool F32>
+template <bool F32, bool STREAM = false>
 __device__ __forceinline__ RopeRow<F32> load_rope_row(const void* src, size_t base) {
   RopeRow<F32> r;
   if constexpr (F32) {
@@ -70,7 +70,8 @@ __device__ __forceinline__ RopeRow<F32> load_rope_row(const void* src, size_t ba
     r.a = *reinterpret_cast<const f32x4*>(p);
     r.b = *reinterpret_cast<const f32x4*>(p + 4);
   } else {
-    r.v = ld_stream<bf16x8>(reinterpret_cast<const bf16*>(src) + base);
+    const bf16* p = reinterpret_cast<const bf16*>(src) + base;
+    r.v = STREAM ? ld_stream<bf16x8>(p) : ld_bf16x8(p);
   }
   return r;
 }
@@ -188,7 +189,7 @@ constexpr int kRopeFwdBatch = 4;
 // them when the q and k heads fill at most four groups) are issued first,
 // the angles are evaluated while they are in flight, then each group is
 // normalised, rotated and stored.
-template <bool F32>
+template <bool F32, bool STREAM>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 3, dl = lane & 7;
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
         size_t base;
         bool live;
         locate(i0 + j, src, dst, base, live);
-        x[j] = load_rope_row<F32>(src, base);
+        x[j] = load_rope_row<F32, STREAM>(src, base);
       }
     }
   };
@@ -385,8 +386,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_bwd_kernel(RopeBwdArgs a) {
           size_t base;
           bool live;
           locate(tok, i0 + j, src, gsrc, dst, base, live);
-          x[j] = load_rope_row<F32>(src, base);
-          go[j] = load_rope_row<F32>(gsrc, base);
+          x[j] = load_rope_row<F32, true>(src, base);
+          go[j] = load_rope_row<F32, true>(gsrc, base);
         }
       }
       // the token's angles, evaluated while its loads are in flight
@@ -500,9 +501,11 @@ hipError_t launch_qk_norm_rope(const void* q, const void* k, const void* q_gain,
   const size_t total = (size_t)B * T;
   const dim3 grid((unsigned)((total + 3) / 4));
   if (f32)
-    hipLaunchKernelGGL((qk_norm_rope_kernel<true>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((qk_norm_rope_kernel<true, false>), grid, dim3(256), 0, stream, a);
+  else if (total * (Hq + Hkv) * kD * (2 * sizeof(bf16)) >= kStreamBytes)
+    hipLaunchKernelGGL((qk_norm_rope_kernel<false, true>), grid, dim3(256), 0, stream, a);
   else
-    hipLaunchKernelGGL((qk_norm_rope_kernel<false>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((qk_norm_rope_kernel<false, false>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
