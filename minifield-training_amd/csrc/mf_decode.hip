@@ -555,6 +555,16 @@ __global__ __launch_bounds__(512) void decode_bf16_kernel(DecArgs a) {
 // the block's (max, sum, acc) go to the partial buffer the combine kernel
 // reads (or, when the cache is one block long, its output to `out`).
 //
+// Probabilities: groups of 1, 2, 4 and 8 heads round them to bf16 for P V (the
+// row sum adds them unrounded).  The other groups, which ran on decode_kernel's
+// fp32 probabilities before they came here, keep them in fp32 (rows_f32_p), so
+// that their error is the output's rounding alone.  Against float64, relative
+// 2-norm, 24/8 heads at 1 x 4096, 40 x 1280 and 128 x 1024: 1.72e-3, 1.67e-3 and
+// 1.66e-3 (decode_kernel the same), with rounded probabilities 1.95e-3, 2.23e-3
+// and 2.33e-3.  It costs 0 to 8 % of the call: 24/8 at 64 x 4096 65.7 -> 63.8 us
+// (decode_kernel: 434), 56/8 at 1 x 4096 21.0 -> 22.7, at 64 x 4096 98.9 -> 105.6,
+// 6/2 at 64 x 8192 35.7 -> 39.4, the largest.
+//
 // Items are 128 tokens of a row; W waves share one.  W = 1: four items a
 // workgroup, numbered by a scan of the lengths so that the grid's first waves
 // are the ones with work: for calls with enough items to keep HBM busy.  Fewer
@@ -604,6 +614,9 @@ template <int G, int TPL>
 constexpr int rows_most_waves() {
   return G == 8 ? (TPL < 8 ? 4 : 2) : TPL == 1 && G > 4 ? 8 : 16 / TPL;
 }
+
+// Groups whose probabilities stay fp32 (see above).
+constexpr bool rows_f32_p(int G) { return (G & (G - 1)) != 0; }
 
 template <int G, int TPL, int W, bool KEEP_V = true>
 __global__ __launch_bounds__((W == 1 ? 256 : 64 * W)) void decode_rows_kernel(DecArgs a) {
@@ -684,6 +697,15 @@ __global__ __launch_bounds__((W == 1 ? 256 : 64 * W)) void decode_rows_kernel(De
       kr[u] = BLOCK ? ld_u32x4(kp) : ld_nt(kp);
       vr[u] = KEEP_V ? ld_u32x4(vp) : ld_nt(vp);
     }
+    if constexpr (rows_f32_p(G)) {
+      // V past the end, which was read again from token `last`, counts as zero:
+      // its probability is 0, and an infinite value must not make 0 * inf of it
+      if (tb + kStep - 1 > last) {
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u)
+          if (tb + j + TPL * u > last) vr[u] = u32x4{0, 0, 0, 0};
+      }
+    }
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       float s[kRowUnroll];
@@ -711,6 +733,18 @@ __global__ __launch_bounds__((W == 1 ? 256 : 64 * W)) void decode_rows_kernel(De
       for (int u = 0; u < kRowUnroll; ++u) {
         p[u] = fast_exp2(s[u] - shift);
         l[g] += p[u];
+      }
+      if constexpr (rows_f32_p(G)) {
+        // P V in fp32, token by token
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t w = vr[u][i];
+            acc[g][2 * i] = fmaf(p[u], __uint_as_float(w << 16), acc[g][2 * i]);
+            acc[g][2 * i + 1] = fmaf(p[u], __uint_as_float(w & 0xffff0000u), acc[g][2 * i + 1]);
+          }
+        continue;
       }
       // P V: bf16 pairs over tokens (u, u + 1)
 #pragma unroll
