@@ -200,8 +200,8 @@ void bwd_dq_f32_kernel(BwdArgs a) {
       continue;
     }
     wave_lds_fence();
-    f32_store(kt[wave], lane, kx);
-    f32_store(vt[wave], lane, vx);
+    f32_store(kt[wave], lane, kx, a.S - kb);
+    f32_store(vt[wave], lane, vx, a.S - kb);
     wave_lds_fence();
     more = fetch(i);
     f32x16 s = zero16(), dp;
@@ -305,7 +305,7 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
   f32x4 qx[8], gx[8];
   int qidl = 0, entry = 0, q0 = 0, head = 0;
   float rowl = 0.f;  // lse2 (lanes of half 0) or -D (half 1) of row q0 + col
-  // the next pair at or after `it` (in steps of 4) that is not wholly before
+  // the next pair at or after `it` (in steps of kKvWaves) that is not wholly before
   // the keys, and its rows; -1 past the list
   auto fetch = [&](int it) {
     for (; it < niters; it += kKvWaves) {
@@ -319,13 +319,13 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
     qidl = qid_row[q0 + col];
     f32_load(qg + head * kRow, q_stride, q0, a.T - 1, lane, qx);
     f32_load(gg + head * kRow, q_stride, q0, a.T - 1, lane, gx);
-    // a row past the end re-reads row T - 1: its id is 0, so its pairs are
-    // masked or belong to an inactive key
+    // (a row past the end: D = 0 and an infinite lse, so P = 0)
     const size_t row = ((size_t)b * a.Hq + head) * a.T;
+    const bool in = q0 + col < a.T;
     const uint32_t at = 4u * (uint32_t)min(q0 + col, a.T - 1);
     const float l2 = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.lse2 + row) + at);
     const float nd = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.ndelta + row) + at);
-    rowl = half ? nd : l2;
+    rowl = half ? (in ? nd : 0.f) : (in ? l2 : kPosInf);
     return it;
   };
   int it = fetch(wave);
@@ -347,8 +347,8 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
     }
     wave_lds_fence();
     rows[wave][half][col] = rowl;
-    f32_store(qt[wave], lane, qx);
-    f32_store(gt[wave], lane, gx);
+    f32_store(qt[wave], lane, qx, a.T - qb);
+    f32_store(gt[wave], lane, gx, a.T - qb);
     wave_lds_fence();
     it = fetch(it + kKvWaves);
     f32x16 s = zero16(), dp;

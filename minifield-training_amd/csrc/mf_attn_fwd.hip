@@ -127,8 +127,8 @@ void attn_fwd_f32_kernel(FwdArgs a) {
       continue;
     }
     wave_lds_fence();
-    f32_store(kt[wave], lane, kx);
-    f32_store(vt[wave], lane, vx);
+    f32_store(kt[wave], lane, kx, a.S - kb);
+    f32_store(vt[wave], lane, vx, a.S - kb);
     wave_lds_fence();
     more = fetch(i);
     f32x16 s = zero16();

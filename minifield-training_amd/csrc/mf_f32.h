@@ -58,7 +58,8 @@ struct F32Tile {
 
 // Rows r0 .. r0 + 31 as loaded: row 4 i + lane / 16, 16-byte piece lane % 16.
 // `base` is wave-uniform, `stride` in bytes; offsets are 32-bit (the entry
-// points reject batch rows of 4 GiB or more).  Rows past `last` re-read it.
+// points reject batch rows of 4 GiB or more).  Rows past `last` re-read it, until
+// f32_store drops them.
 __device__ __forceinline__ void f32_load(const char* base, uint32_t stride, int r0, int last,
                                          int lane, f32x4 (&x)[8]) {
   if (r0 + 31 <= last) {
@@ -76,7 +77,16 @@ __device__ __forceinline__ void f32_load(const char* base, uint32_t stride, int 
   }
 }
 
-__device__ __forceinline__ void f32_store(F32Tile& t, int lane, const f32x4 (&x)[8]) {
+// Rows `rows` and on of the block lie past the sequence end and are stored as
+// zero: their probabilities are zero, and 0 * inf must not come of a row that
+// was read in their place.  (Here, not at the loads, which stay in flight.)
+__device__ __forceinline__ void f32_store(F32Tile& t, int lane, f32x4 (&x)[8],
+                                          int rows = 32) {
+  if (rows < 32) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (4 * i + (lane >> 4) >= rows) x[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     *reinterpret_cast<f32x4*>(&t.x[(4 * i + (lane >> 4)) * kF32Pitch + 4 * (lane & 15)]) = x[i];
