@@ -52,6 +52,7 @@ struct BwdArgs {
   int fuse_delta;  // dq computes D = rowsum(dO * O) itself and writes -D and lse2
   float scale, scale_log2;
   FastDiv div_nh, div_hchunks, div_nq, div_hkv, div_nk, div_g, div_hq;  // Hkv * hchunks, hchunks, nq, Hkv, nk, G, Hq
+  FastDiv div_qsub, div_ksub;  // row blocks per query and key tile (fp32 units)
 };
 
 constexpr int kStep = 64;
@@ -111,7 +112,7 @@ void bwd_dq_f32_kernel(BwdArgs a) {
   const int wave = uniform(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
   F32Unit w;
-  if (!f32_unit(a.qorder, a.div_hq, a.div_hkv, a.div_nq, a.T, a.G, w)) return;
+  if (!f32_unit(a.qorder, a.div_hq, a.div_hkv, a.div_qsub, a.div_nq, a.T, a.G, w)) return;
   const int b = w.b, q0 = w.row0;
   const int qpos = q0 + col;
   const int qrow = min(qpos, a.T - 1);
@@ -276,7 +277,7 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
   const int wave = uniform(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
   F32Unit w;
-  if (!f32_unit(a.korder, a.div_hkv, a.div_hkv, a.div_nk, a.S, 1, w)) return;
+  if (!f32_unit(a.korder, a.div_hkv, a.div_hkv, a.div_ksub, a.div_nk, a.S, 1, w)) return;
   const int b = w.b, k0 = w.row0, kvh = w.kvh;
   const int kpos = k0 + col;
   const int mykid = a.kid[(size_t)b * a.tk_pad + kpos];
@@ -988,6 +989,8 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   a.div_nk = make_fastdiv(a.nk);
   a.div_g = make_fastdiv(a.G);
   a.div_hq = make_fastdiv(Hq);
+  a.div_qsub = make_fastdiv(f32_blocks(T));
+  a.div_ksub = make_fastdiv(f32_blocks(S));
   const size_t rows = (size_t)batch * T * Hq;
   const unsigned dgrid = (unsigned)((rows + 255) / 256);
   // with both the delta and the dq phase the dq kernel, which holds the dO
@@ -1003,7 +1006,8 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   const dim3 qgrid(Hkv * a.hchunks * batch * lay.nq);
   if (!(phases & 2)) {
   } else if (f32) {
-    hipLaunchKernelGGL(bwd_dq_f32_kernel, dim3(4 * Hq * batch * lay.nq), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(bwd_dq_f32_kernel, dim3(f32_blocks(T) * Hq * batch * lay.nq), dim3(256), 0,
+                       stream, a);
   } else {
     if (hpw == 2)
       hipLaunchKernelGGL((bwd_dq_bf16_kernel<2>), qgrid, dim3(512), 0, stream, a);
@@ -1016,7 +1020,8 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
     // C2/C3/C5 than 8-wave workgroups whose halves took different heads and
     // summed through LDS, because the workgroups of a CU share no barriers.
     if (f32)
-      hipLaunchKernelGGL(bwd_dkdv_f32_kernel, dim3(4 * Hkv * batch * lay.nk), dim3(64 * kKvWaves), 0, stream, a);
+      hipLaunchKernelGGL(bwd_dkdv_f32_kernel, dim3(f32_blocks(S) * Hkv * batch * lay.nk),
+                         dim3(64 * kKvWaves), 0, stream, a);
     else
       hipLaunchKernelGGL(bwd_dkdv_bf16_kernel, kgrid, dim3(256), 0, stream, a);
   }

@@ -32,7 +32,7 @@ struct FwdArgs {
   int causal;
   float scale, scale_log2;
   FastDiv div_nh, div_hchunks, div_nq;  // Hkv * hchunks, hchunks, nq
-  FastDiv div_hq, div_hkv;              // Hq, Hkv (fp32 units)
+  FastDiv div_hq, div_hkv, div_qsub;    // Hq, Hkv, row blocks per tile (fp32 units)
   // query prologue fused into the bf16 kernel's query loads (ROPE instances)
   const void* q_gain;           // [64], tensor dtype
   const int32_t* positions;     // [B, T] or null (0 .. T-1 on every row)
@@ -67,7 +67,7 @@ void attn_fwd_f32_kernel(FwdArgs a) {
   const int wave = uniform(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
   F32Unit w;
-  if (!f32_unit(a.qorder, a.div_hq, a.div_hkv, a.div_nq, a.T, a.G, w)) return;
+  if (!f32_unit(a.qorder, a.div_hq, a.div_hkv, a.div_qsub, a.div_nq, a.T, a.G, w)) return;
   const int b = w.b, q0 = w.row0, kvh = w.kvh, head = w.head;
   const int qpos = q0 + col;
   const int myqid = a.qid[(size_t)b * a.tq_pad + qpos];
@@ -613,6 +613,7 @@ static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, 
   a.div_nq = make_fastdiv(a.nq);
   a.div_hq = make_fastdiv(Hq);
   a.div_hkv = make_fastdiv(Hkv);
+  a.div_qsub = make_fastdiv(f32_blocks(T));
   return a;
 }
 
@@ -623,7 +624,8 @@ hipError_t launch_attn_fwd(const void* q, const void* k, const void* v, bool f32
   const FwdArgs a = fwd_args(q, k, v, batch, T, S, Hq, Hkv, mode, scale, plan, out, lse, &hpw);
   const dim3 grid(Hkv * a.hchunks * batch * a.nq);
   if (f32) {
-    hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(4 * Hq * batch * a.nq), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(f32_blocks(T) * Hq * batch * a.nq), dim3(256), 0,
+                       stream, a);
   } else {
     if (hpw == 2)
       hipLaunchKernelGGL((attn_fwd_bf16_kernel<2, false>), grid, dim3(512), 0, stream, a);

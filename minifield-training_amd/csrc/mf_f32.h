@@ -13,23 +13,32 @@ struct F32Unit {
   int b, tile, row0, kvh, head;
 };
 
+// 32-row blocks a launch has per tile: all four, unless the one tile of a
+// shorter row has fewer.  With four, most workgroups of such a row are empty; us,
+// forward and backward, four -> fewer: 4096 x 8, 4/4 heads 840 and 3128 -> 234 and
+// 819; 512 x 24, 16/8 heads 214 and 807 -> 120 and 300; 512 x 90 492 and 1495 ->
+// 387 and 1154.  (128-row tiles took 370 and 1560, 219 and 725, 491 and 1762.)
+inline int f32_blocks(int len) { return len > 96 ? 4 : (len + 31) / 32; }
+
 // blockIdx.x -> unit: (launch slot, 32-row block of the tile, head), the KV
 // head fastest, so that with 8 KV heads each XCD's L2 holds one head's
 // operands.  `div_h` is the number of heads the grid has per row block (Hq,
-// or Hkv for the key side, where g_heads is 1).  False for a block past the
-// sequence end.
+// or Hkv for the key side, where g_heads is 1), `div_sub` the blocks it has per
+// tile (f32_blocks).  False for a block past the sequence end.
 __device__ __forceinline__ bool f32_unit(const int* order, const FastDiv& div_h,
-                                         const FastDiv& div_hkv, const FastDiv& div_tiles, int len,
-                                         int g_heads, F32Unit& w) {
+                                         const FastDiv& div_hkv, const FastDiv& div_sub,
+                                         const FastDiv& div_tiles, int len, int g_heads,
+                                         F32Unit& w) {
   const int blk = uniform(fast_div(blockIdx.x, div_h));
   const int h = uniform(blockIdx.x - blk * (int)div_h.d);
   const int g = uniform(fast_div(h, div_hkv));
   w.kvh = uniform(h - g * (int)div_hkv.d);
   w.head = w.kvh * g_heads + g;
-  const int item = ld_const(order, blk >> 2);
+  const int slot = uniform(fast_div(blk, div_sub));
+  const int item = ld_const(order, slot);
   w.b = uniform(fast_div(item, div_tiles));
   w.tile = uniform(item - w.b * (int)div_tiles.d);
-  w.row0 = w.tile * kTile + 32 * (blk & 3);
+  w.row0 = w.tile * kTile + 32 * (blk - slot * (int)div_sub.d);
   return w.row0 < len;
 }
 
