@@ -1006,8 +1006,11 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   const dim3 qgrid(Hkv * a.hchunks * batch * lay.nq);
   if (!(phases & 2)) {
   } else if (f32) {
-    hipLaunchKernelGGL(bwd_dq_f32_kernel, dim3(f32_blocks(T) * Hq * batch * lay.nq), dim3(256), 0,
-                       stream, a);
+    f32_launch(a.qorder, (size_t)batch * lay.nq, (size_t)f32_blocks(T) * Hq, 256,
+               [&](const int* order, unsigned blocks) {
+                 a.qorder = order;
+                 hipLaunchKernelGGL(bwd_dq_f32_kernel, dim3(blocks), dim3(256), 0, stream, a);
+               });
   } else {
     if (hpw == 2)
       hipLaunchKernelGGL((bwd_dq_bf16_kernel<2>), qgrid, dim3(512), 0, stream, a);
@@ -1020,8 +1023,12 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
     // C2/C3/C5 than 8-wave workgroups whose halves took different heads and
     // summed through LDS, because the workgroups of a CU share no barriers.
     if (f32)
-      hipLaunchKernelGGL(bwd_dkdv_f32_kernel, dim3(f32_blocks(S) * Hkv * batch * lay.nk),
-                         dim3(64 * kKvWaves), 0, stream, a);
+      f32_launch(a.korder, (size_t)batch * lay.nk, (size_t)f32_blocks(S) * Hkv, 64 * kKvWaves,
+                 [&](const int* order, unsigned blocks) {
+                   a.korder = order;
+                   hipLaunchKernelGGL(bwd_dkdv_f32_kernel, dim3(blocks), dim3(64 * kKvWaves), 0,
+                                      stream, a);
+                 });
     else
       hipLaunchKernelGGL(bwd_dkdv_bf16_kernel, kgrid, dim3(256), 0, stream, a);
   }

@@ -621,11 +621,14 @@ hipError_t launch_attn_fwd(const void* q, const void* k, const void* v, bool f32
                            int T, int S, int Hq, int Hkv, int mode, float scale,
                            const void* plan, void* out, float* lse, hipStream_t stream) {
   int hpw;
-  const FwdArgs a = fwd_args(q, k, v, batch, T, S, Hq, Hkv, mode, scale, plan, out, lse, &hpw);
+  FwdArgs a = fwd_args(q, k, v, batch, T, S, Hq, Hkv, mode, scale, plan, out, lse, &hpw);
   const dim3 grid(Hkv * a.hchunks * batch * a.nq);
   if (f32) {
-    hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(f32_blocks(T) * Hq * batch * a.nq), dim3(256), 0,
-                       stream, a);
+    f32_launch(a.qorder, (size_t)batch * a.nq, (size_t)f32_blocks(T) * Hq, 256,
+               [&](const int* order, unsigned blocks) {
+                 a.qorder = order;
+                 hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(blocks), dim3(256), 0, stream, a);
+               });
   } else {
     if (hpw == 2)
       hipLaunchKernelGGL((attn_fwd_bf16_kernel<2, false>), grid, dim3(512), 0, stream, a);

@@ -20,6 +20,17 @@ struct F32Unit {
 // 387 and 1154.  (128-row tiles took 370 and 1560, 219 and 725, 491 and 1762.)
 inline int f32_blocks(int len) { return len > 96 ? 4 : (len + 31) / 32; }
 
+// Launches `launch(order, grid)` for `items` tiles in launch order, `per_item`
+// workgroups of `threads` each, in as many pieces as the limit of 2^32 - 1 threads
+// per launch asks for (one piece up to 2^31 threads).
+template <typename L>
+inline void f32_launch(const int* order, size_t items, size_t per_item, int threads, L launch) {
+  size_t piece = ((size_t)1 << 31) / (per_item * threads);
+  if (piece < 1) piece = 1;
+  for (size_t at = 0; at < items; at += piece)
+    launch(order + at, (unsigned)(per_item * (items - at < piece ? items - at : piece)));
+}
+
 // blockIdx.x -> unit: (launch slot, 32-row block of the tile, head), the KV
 // head fastest, so that with 8 KV heads each XCD's L2 holds one head's
 // operands.  `div_h` is the number of heads the grid has per row block (Hq,

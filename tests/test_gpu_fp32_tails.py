@@ -31,3 +31,22 @@ def test_an_infinite_last_row_stays_infinite(t, device):
     inf[0, :, 2:, 3] = True
     assert (out[inf] == float("inf")).all() and torch.isfinite(out[~inf]).all()
     assert torch.isfinite(lse).all()
+
+
+def test_more_workgroups_than_one_launch_may_have(device):
+    """65535 rows of one token, 260/130 heads: the forward, dq and dk/dv each exceed 2**32 threads,
+    the limit of one launch.  A row that sees one key copies it: out is the value of each head's
+    group, dq and dk are zero and dv sums the group's gradients."""
+    rows, hq, hkv = 65535, 260, 130
+    gen = torch.Generator(device=device).manual_seed(1)
+    q, k, v, do = (torch.randn((rows, 1, h, 64), generator=gen, device=device)
+                   for h in (hq, hkv, hkv, hq))
+    seg = torch.ones((rows, 1), dtype=torch.int32, device=device)
+    plan = ops.block_map(seg, seg, 0, 1, 1)
+    out, lse = ops.attn_fwd(q, k, v, plan, 0, 0.125)
+    # softmax of one score is 1: exp2 of a rounding error (2**-21 of a score below 16), times 1 / l
+    assert torch.allclose(out, v.repeat_interleave(2, dim=2), rtol=1e-5, atol=1e-5)
+    dq, dk, dv = ops.attn_bwd(q, k, v, out, do, lse, plan, 0, 0.125)
+    assert torch.allclose(dv, do.view(rows, 1, hkv, 2, 64).sum(3), rtol=1e-5, atol=2e-5)
+    # dS = P (dP - D): dP and D are the same 64 products in another order
+    assert dq.abs().max() < 1e-4 and dk.abs().max() < 1e-4
