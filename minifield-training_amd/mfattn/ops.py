@@ -21,8 +21,10 @@ _DTYPES = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
 
 
 # The current stream's handle by device index.  torch.cuda.current_stream
-# builds a Stream object for the same number (1.9 us against 0.1).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# builds a Stream object for the same number (1.9 us against 0.1); it serves a
+# torch without the private query (a build for the CPU has none).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _stream(device: torch.device) -> int:

@@ -7,6 +7,10 @@ shapes (the block map reads B x S mask entries and B x T ids, and the plan is
 indexed with the query's batch), and plans built for another call.
 """
 
+import pathlib
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -132,3 +136,28 @@ def test_strided_views_are_refused_before_any_launch():
                           torch.zeros_like(k), torch.zeros_like(v))
     with pytest.raises(ValueError, match="lse must be"):
         ops.attn_bwd_delta(out, torch.zeros_like(q), torch.zeros(2, 4, 15), ws)
+
+
+def test_a_torch_without_the_raw_stream_query_still_imports():
+    """torch._C._cuda_getCurrentRawStream is private and absent from a CPU build: the package
+    imports without it and refuses host tensors as ever; on a GPU the public query stands in."""
+    code = """
+import sys, types, torch
+sys.path.insert(0, sys.argv[1])
+if hasattr(torch._C, "_cuda_getCurrentRawStream"):
+    del torch._C._cuda_getCurrentRawStream
+from mfattn import ops
+x = torch.zeros(2, 1, 4, 64)
+try:
+    ops.decode(x, torch.zeros(2, 16, 2, 64), torch.zeros(2, 16, 2, 64),
+               torch.ones(2, dtype=torch.int32), 1.0)
+except ValueError as exc:
+    assert "runs on the GPU only" in str(exc), exc
+else:
+    raise SystemExit("host tensors were accepted")
+torch.cuda.current_stream = lambda device: types.SimpleNamespace(cuda_stream=40 + device)
+assert ops._stream(torch.device("cuda", 2)) == 42
+"""
+    package = pathlib.Path(ops.__file__).resolve().parents[1]
+    proc = subprocess.run([sys.executable, "-c", code, str(package)], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr
