@@ -63,19 +63,18 @@ class QKNormRope(torch.autograd.Function):
         dk_out = torch.zeros_like(k) if dk_out is None else dk_out.contiguous()
         dq, dk = torch.empty_like(q), torch.empty_like(k)
         b, t, hq, d = q.shape
-        # both gain gradients in one buffer, cast to the gains' dtype (the
-        # tensors') by one launch
-        dgains = torch.empty((2, d), dtype=torch.float32, device=q.device)
-        dqg = dgains.data_ptr()
+        # one buffer each: a gradient that is a view of a shared one counts as
+        # modified whenever the other is
+        dqg = torch.empty(d, dtype=torch.float32, device=q.device)
+        dkg = torch.empty_like(dqg)
         ws_bytes = _lib.LIB.mf_qk_norm_rope_bwd_workspace_bytes(b, t)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
         _lib.check(_lib.LIB.mf_qk_norm_rope_bwd(
             _ptr(q), _ptr(k), _ptr(qg), _ptr(kg), _ptr(pos), _ptr(dq_out), _ptr(dk_out),
             dtype_code(q), b, t, hq, k.shape[2], d, float(ctx.eps),
-            float(ctx.theta), _ptr(dq), _ptr(dk), dqg, dqg + 4 * d, _ptr(ws), ws_bytes,
+            float(ctx.theta), _ptr(dq), _ptr(dk), _ptr(dqg), _ptr(dkg), _ptr(ws), ws_bytes,
             _stream(q.device)))
-        dgains = dgains.to(qg.dtype)
-        return dq, dk, dgains[0], dgains[1], None, None, None
+        return dq, dk, dqg.to(qg.dtype), dkg.to(kg.dtype), None, None, None
 
 
 def qk_norm_rope(query: torch.Tensor, key: torch.Tensor, query_gain: torch.Tensor,

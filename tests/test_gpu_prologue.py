@@ -268,3 +268,20 @@ def test_large_positions_and_head_counts(hq, hkv, device):
     for name, a, r in zip(("q", "k", "dq", "dk", "dq_gain", "dk_gain"), got, (rq, rk, *vjp)):
         scale = max(1.0, float(np.abs(r).max()))
         np.testing.assert_allclose(a.detach().cpu().numpy(), r, rtol=1e-5, atol=1e-5 * scale, err_msg=name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gain_gradients_are_tensors_of_their_own(dtype, device):
+    """The two gain gradients share neither memory nor a version counter: changing one in place
+    (clipping, an optimizer) leaves the other unmodified for autograd."""
+    gen = torch.Generator(device=device).manual_seed(3)
+    q, k = (torch.randn((1, 40, h, 64), generator=gen, device=device).to(dtype) for h in (4, 2))
+    gains = [torch.ones(64, device=device, dtype=dtype, requires_grad=True) for _ in range(2)]
+    out = prologue.qk_norm_rope(q, k, *gains, None, eps=1e-5, rope_theta=1e4)
+    a, b = torch.autograd.grad(out, gains, [torch.ones_like(x) for x in out])
+    assert a.untyped_storage().data_ptr() != b.untyped_storage().data_ptr()
+    assert a.untyped_storage().nbytes() == b.untyped_storage().nbytes() == a.nbytes
+    assert a._base is None and b._base is None
+    before = b._version
+    a.mul_(0.5)
+    assert b._version == before
