@@ -173,6 +173,11 @@ __device__ __forceinline__ u32x4 ld_u32x4(const void* p) {
 // us, 201 MB 39.6 and 36.2; conv, 269 MB, 47.9 and 43.2.
 constexpr size_t kStreamBytes = (size_t)128 << 20;
 
+// The same of a backward pass, whose gradient has just been made and whose
+// results are read next: about what the last-level cache holds (256 MB).
+// Figures at the kernels (conv_bwd_tile, qk_norm_rope_bwd_kernel).
+constexpr size_t kStreamBwdBytes = (size_t)256 << 20;
+
 // Accesses to data that one pass streams through once (no reuse in L2).
 template <typename V>
 __device__ __forceinline__ V ld_stream(const void* p) {

@@ -258,44 +258,48 @@ constexpr int conv_bwd_channels() {
   return K <= 4 || (K == 5 && CENTERED && !std::is_same<T, float>::value) ? 8 : 4;
 }
 
-// CW elements of one token row of the backward as loaded.
+// CW elements of one token row of the backward as loaded (rows of four channels
+// are never streamed: their windows are too wide).
 template <typename T, int CW, bool STREAM>
 struct RawC : Raw8<T, STREAM> {};
-template <bool STREAM>
-struct RawC<bf16, 4, STREAM> {
+template <>
+struct RawC<bf16, 4, false> {
   bf16x4 v;
   __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const bf16x4*>(p); }
   __device__ __forceinline__ float operator[](int e) const { return (float)v[e]; }
 };
-template <bool STREAM>
-struct RawC<float, 4, STREAM> {
+template <>
+struct RawC<float, 4, false> {
   f32x4 v;
   __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const f32x4*>(p); }
   __device__ __forceinline__ float operator[](int e) const { return v[e]; }
 };
 
-// The backward's gradients go out as streams (nothing of the call reads them
-// again): forward and backward of 4 x 4096 x 768 fp32, K = 4, 152 -> 147.4 us,
-// 8 x 4096 x 1024 bf16, K = 4, 232 -> 228.  A consumer that reads all of them
-// right away finds less of them cached: 64 x 512 x 512 with such a pass
-// 148.3 -> 150.3, 8 x 4096 x 1024 259 -> 257, streamed loads included.
-template <typename T, int CW>
+// STREAM: the gradients go out as streams (nothing of the call reads them
+// again); launch_conv_bwd_t has the line and what it measures.
+template <bool STREAM, typename V>
+__device__ __forceinline__ void st_maybe_stream(void* p, const V& v) {
+  if constexpr (STREAM) st_stream(p, v);
+  else *reinterpret_cast<V*>(p) = v;
+}
+
+template <typename T, int CW, bool STREAM>
 __device__ __forceinline__ void store_row(T* p, const float (&x)[CW]) {
   if constexpr (std::is_same<T, float>::value) {
 #pragma unroll
     for (int h = 0; h < CW; h += 4) {
       const f32x4 v = {x[h], x[h + 1], x[h + 2], x[h + 3]};
-      st_stream(p + h, v);
+      st_maybe_stream<STREAM>(p + h, v);
     }
   } else if constexpr (CW == 8) {
     uint32_t words[4];
 #pragma unroll
     for (int e = 0; e < 8; e += 2) words[e / 2] = pack_pair(x[e], x[e + 1]);
     const u32x4 v = {words[0], words[1], words[2], words[3]};
-    st_stream(p, v);
+    st_maybe_stream<STREAM>(p, v);
   } else {
     const u32x2 v = {pack_pair(x[0], x[1]), pack_pair(x[2], x[3])};
-    st_stream(p, v);
+    st_maybe_stream<STREAM>(p, v);
   }
 }
 
@@ -306,7 +310,7 @@ __device__ __forceinline__ void store_row(T* p, const float (&x)[CW]) {
 // width) kAhead steps before it is used; at step q output q - (W - 1) is
 // formed from the W newest slots, so every row is loaded once per thread.
 // The step loop is unrolled by R, so all slot indices are compile-time.
-template <typename T, int K, int LO, int CW>
+template <typename T, int K, int LO, int CW, bool STREAM>
 __device__ __forceinline__ void conv_bwd_tile(const ConvBwdArgs& a, size_t row, int t0, int c0,
                                               const float (&w)[K][CW], float (&dw)[K][CW]) {
   constexpr bool kBf16 = !std::is_same<T, float>::value;
@@ -320,13 +324,14 @@ __device__ __forceinline__ void conv_bwd_tile(const ConvBwdArgs& a, size_t row, 
   const T* bp = reinterpret_cast<const T*>(a.b);
   const T* cp = reinterpret_cast<const T*>(a.c);
   const T* gp = reinterpret_cast<const T*>(a.g);
-  // A tile re-reads W - 1 of its neighbour's rows.  Up to W = 5 its loads still
-  // gain as streams, at W = 7 no longer.  us, forward and backward, without
+  // A tile re-reads W - 1 of its neighbour's rows.  Up to W = 5 its bf16 loads
+  // still gain as streams, at W = 7 no longer.  us, forward and backward, without
   // and with (stores as streams on both sides): 8 x 4096 x 1024 bf16, W = 3
   // 175 -> 168, W = 5 180.7 -> 176.5; 8 x 4096 x 768, W = 5 161.5 -> 156;
   // 9 x 1777 x 768, W = 7 119.5 -> 122
-  constexpr bool kStream = W <= 5;
-  RawC<T, CW, kStream> rv[R], rb[R], rg[R], rc[R];
+  constexpr bool kStreamLoads = STREAM && kBf16 && W <= 5;
+  static_assert(!kStreamLoads || CW == 8, "");
+  RawC<T, CW, kStreamLoads> rv[R], rb[R], rg[R], rc[R];
   int sg[R];
   auto issue = [&](int q, int slot) {
     const int s = t0 + SMIN + q;
@@ -389,24 +394,24 @@ __device__ __forceinline__ void conv_bwd_tile(const ConvBwdArgs& a, size_t row, 
         float dc[CW];
 #pragma unroll
         for (int e = 0; e < CW; ++e) dc[e] = rg[s0][e] * m[e];
-        store_row<T, CW>(reinterpret_cast<T*>(a.dc) + off, dc);
+        store_row<T, CW, STREAM>(reinterpret_cast<T*>(a.dc) + off, dc);
       }
       float dv[CW];
       if (a.b) {
         float db[CW];
 #pragma unroll
         for (int e = 0; e < CW; ++e) dv[e] = du[e] * rb[s0][e], db[e] = du[e] * rv[s0][e];
-        store_row<T, CW>(reinterpret_cast<T*>(a.db) + off, db);
+        store_row<T, CW, STREAM>(reinterpret_cast<T*>(a.db) + off, db);
       } else {
 #pragma unroll
         for (int e = 0; e < CW; ++e) dv[e] = du[e];
       }
-      store_row<T, CW>(reinterpret_cast<T*>(a.dv) + off, dv);
+      store_row<T, CW, STREAM>(reinterpret_cast<T*>(a.dv) + off, dv);
     }
   }
 }
 
-template <typename T, int K, bool CENTERED>
+template <typename T, int K, bool CENTERED, bool STREAM>
 __global__ __launch_bounds__(256) void segmented_conv_bwd_kernel(ConvBwdArgs a) {
   constexpr int CW = conv_bwd_channels<T, K, CENTERED>();
   __shared__ float red[4][kConvBwdChunks][K * CW];
@@ -437,7 +442,7 @@ __global__ __launch_bounds__(256) void segmented_conv_bwd_kernel(ConvBwdArgs a) 
 
   if (on) {
     const int t0 = tile * kConvBwdTile;
-    conv_bwd_tile<T, K, CENTERED ? -(K / 2) : -(K - 1), CW>(a, row, t0, c0, w, dw);
+    conv_bwd_tile<T, K, CENTERED ? -(K / 2) : -(K - 1), CW, STREAM>(a, row, t0, c0, w, dw);
   }
   // tap gradients: add the 8 tiles of each wave (lanes lc, lc + 8, ... hold
   // the same channels), then the 4 waves, in a fixed order
@@ -503,16 +508,30 @@ hipError_t launch_conv_bwd_t(const ConvBwdArgs& a, hipStream_t stream) {
     const int chunks = a.C / cw;
     return dim3((unsigned)(a.B * tgroups * ((chunks + kConvBwdChunks - 1) / kConvBwdChunks)));
   };
-#define MF_CONV_BWD_CASE(KK)                                                                     \
-    case KK: {                                                                                    \
-      if (a.centered)                                                                             \
-        hipLaunchKernelGGL((segmented_conv_bwd_kernel<T, KK, true>),                              \
-                           grid_for(conv_bwd_channels<T, KK, true>()), dim3(256), 0, stream, a);  \
-      else                                                                                        \
-        hipLaunchKernelGGL((segmented_conv_bwd_kernel<T, KK, false>),                             \
-                           grid_for(conv_bwd_channels<T, KK, false>()), dim3(256), 0, stream, a); \
-      break;                                                                                      \
-    }
+  // Accesses as streams from kStreamBwdBytes of inputs and gradients on; below,
+  // dout is still cached from its producer, and the gradients stay cached for
+  // their consumers.  us with a producer of dout before and a consumer of every
+  // gradient behind, cached and streamed, bf16, K = 3 centered: 28 MiB 46.4 and
+  // 49.4, 112 MiB 61.4 and 71.8, 224 MiB 108.6 and 112.1, 336 MiB 178.3 and
+  // 179.0, 448 MiB 222.3 and 214.1, 896 MiB 408.8 and 401.7 (producers of every
+  // input too: 28 MiB 56.3 and 54.4, 112 MiB 80.5 and 86.3, 224 MiB 164.9 and
+  // 152.1, 336 MiB 236.8 and 238.8, 448 MiB 293.2 and 281.2).  Wider filters
+  // than four taps stay cached.
+  const size_t tensors = 3 + 2 * (a.b != nullptr) + 2 * (a.c != nullptr);
+  const bool big = (size_t)a.B * a.T * a.C * sizeof(T) * tensors >= kStreamBwdBytes;
+#define MF_CONV_BWD_LAUNCH(KK, CC, SS)                                                            \
+  hipLaunchKernelGGL((segmented_conv_bwd_kernel<T, KK, CC, SS>),                                  \
+                     grid_for(conv_bwd_channels<T, KK, CC>()), dim3(256), 0, stream, a)
+#define MF_CONV_BWD_CASE(KK)                                                                      \
+    case KK:                                                                                      \
+      if (a.centered) {                                                                           \
+        if (big && KK <= 4) MF_CONV_BWD_LAUNCH(KK, true, KK <= 4);                                \
+        else MF_CONV_BWD_LAUNCH(KK, true, false);                                                 \
+      } else {                                                                                    \
+        if (big && KK <= 4) MF_CONV_BWD_LAUNCH(KK, false, KK <= 4);                               \
+        else MF_CONV_BWD_LAUNCH(KK, false, false);                                                \
+      }                                                                                           \
+      break;
   switch (a.K) {
     MF_CONV_BWD_CASE(1)
     MF_CONV_BWD_CASE(2)
@@ -523,6 +542,7 @@ hipError_t launch_conv_bwd_t(const ConvBwdArgs& a, hipStream_t stream) {
     MF_CONV_BWD_CASE(7)
     MF_CONV_BWD_CASE(8)
 #undef MF_CONV_BWD_CASE
+#undef MF_CONV_BWD_LAUNCH
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
