@@ -175,7 +175,7 @@ constexpr size_t kStreamBytes = (size_t)128 << 20;
 
 // The same of a backward pass, whose gradient has just been made and whose
 // results are read next: about what the last-level cache holds (256 MB).
-// Figures at the kernels (conv_bwd_tile, qk_norm_rope_bwd_kernel).
+// Figures at launch_conv_bwd_t and launch_qk_norm_rope_bwd.
 constexpr size_t kStreamBwdBytes = (size_t)256 << 20;
 
 // Accesses to data that one pass streams through once (no reuse in L2).

@@ -56,12 +56,13 @@ template <bool F32> struct RopeRow;
 template <> struct RopeRow<false> { bf16x8 v; };
 template <> struct RopeRow<true> { f32x4 a, b; };
 
-// STREAM: bf16 rows are read (the backward's also written) as streams, in the
-// forward from kStreamBytes on: every row is touched once, whole 128-byte lines per instruction.  24 x 4096 tokens of
-// 16/8 heads, forward and backward: 291 -> 279 us; the forward alone at
-// 8 x 4096: 39 -> 36.  fp32 keeps plain accesses (a line is touched by two
-// loads of 16 bytes per lane; streamed, the backward takes 70 us against 63),
-// and the forward keeps plain stores (36.4 us both ways).
+// STREAM: bf16 rows are read, and the backward's written, as streams: every row
+// is touched once, whole 128-byte lines per instruction.  The launchers have the
+// lines (kStreamBytes, kStreamBwdBytes).  24 x 4096 tokens of 16/8 heads, forward
+// and backward: 291 -> 279 us; the forward alone at 8 x 4096: 39 -> 36.  fp32 keeps
+// plain accesses (a line is touched by two loads of 16 bytes per lane; streamed,
+// the backward takes 70 us against 63), and the forward keeps plain stores (36.4
+// us both ways).
 template <bool F32, bool STREAM = false>
 __device__ __forceinline__ RopeRow<F32> load_rope_row(const void* src, size_t base) {
   RopeRow<F32> r;
@@ -291,7 +292,7 @@ constexpr int kRopeBatch = 3;          // (token, head group) rows loaded before
 // The VJP of one loaded group: lane (g, dl) holds dims 8 dl .. 8 dl + 7 of
 // head g.  Every lane takes part (shuffles and the 8-lane sums); only live
 // lanes store and accumulate the gain gradient.
-template <bool F32>
+template <bool F32, bool STREAM>
 __device__ __forceinline__ void norm_rope_bwd_store(const RopeRow<F32>& xin,
                                                     const RopeRow<F32>& gin, void* dst,
                                                     size_t base, bool live, const float (&w)[8],
@@ -331,7 +332,9 @@ __device__ __forceinline__ void norm_rope_bwd_store(const RopeRow<F32>& xin,
     bf16x8 o;
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = (bf16)(inv * fmaf(-y[i], mean, dy[i]));
-    st_stream(reinterpret_cast<bf16*>(dst) + base, o);
+    bf16* const to = reinterpret_cast<bf16*>(dst) + base;
+    if constexpr (STREAM) st_stream(to, o);
+    else *reinterpret_cast<bf16x8*>(to) = o;
   }
 }
 
@@ -344,7 +347,7 @@ __device__ __forceinline__ float heads_sum8(float x) {
   return x;
 }
 
-template <bool F32>
+template <bool F32, bool STREAM>
 __global__ __launch_bounds__(256) void qk_norm_rope_bwd_kernel(RopeBwdArgs a) {
   __shared__ float part[4][2][kD];
   const int lane = threadIdx.x & 63;
@@ -386,8 +389,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_bwd_kernel(RopeBwdArgs a) {
           size_t base;
           bool live;
           locate(tok, i0 + j, src, gsrc, dst, base, live);
-          x[j] = load_rope_row<F32, true>(src, base);
-          go[j] = load_rope_row<F32, true>(gsrc, base);
+          x[j] = load_rope_row<F32, STREAM>(src, base);
+          go[j] = load_rope_row<F32, STREAM>(gsrc, base);
         }
       }
       // the token's angles, evaluated while its loads are in flight
@@ -401,9 +404,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_bwd_kernel(RopeBwdArgs a) {
           bool live;
           locate(tok, i0 + j, src, gsrc, dst, base, live);
           if (i0 + j < gq)
-            norm_rope_bwd_store<F32>(x[j], go[j], dst, base, live, wq, c, s, dl, a.eps, dwq);
+            norm_rope_bwd_store<F32, STREAM>(x[j], go[j], dst, base, live, wq, c, s, dl, a.eps, dwq);
           else
-            norm_rope_bwd_store<F32>(x[j], go[j], dst, base, live, wk, c, s, dl, a.eps, dwk);
+            norm_rope_bwd_store<F32, STREAM>(x[j], go[j], dst, base, live, wk, c, s, dl, a.eps, dwk);
         }
       }
     }
@@ -542,10 +545,17 @@ hipError_t launch_qk_norm_rope_bwd(const void* q, const void* k, const void* q_g
   a.eps = eps;
   for (int i = 0; i < kD / 2; ++i) a.freq[i] = powf(theta, -((float)(2 * i) / (float)kD));
   const int blocks = (int)rope_bwd_blocks(B, T);
+  // Streamed from kStreamBwdBytes of rows, gradients and results on.  us with a
+  // producer of the output gradients before and a consumer of the results behind,
+  // cached and streamed, bf16, 16/8 heads: 72 MiB 40.6 and 44.0, 144 MiB 66.0 and
+  // 71.2, 288 MiB 134.8 and 131.6, 864 MiB 387.5 and 370.5.
+  const size_t bytes = (size_t)B * T * (Hq + Hkv) * kD * (3 * sizeof(bf16));
   if (f32)
-    hipLaunchKernelGGL((qk_norm_rope_bwd_kernel<true>), dim3(blocks), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((qk_norm_rope_bwd_kernel<true, false>), dim3(blocks), dim3(256), 0, stream, a);
+  else if (bytes >= kStreamBwdBytes)
+    hipLaunchKernelGGL((qk_norm_rope_bwd_kernel<false, true>), dim3(blocks), dim3(256), 0, stream, a);
   else
-    hipLaunchKernelGGL((qk_norm_rope_bwd_kernel<false>), dim3(blocks), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((qk_norm_rope_bwd_kernel<false, false>), dim3(blocks), dim3(256), 0, stream, a);
   hipLaunchKernelGGL(rope_gain_reduce_kernel, dim3(2 * kD), dim3(kRopeReduceThreads), 0, stream,
                      a.partials, blocks, dq_gain, dk_gain);
   return hipGetLastError();
