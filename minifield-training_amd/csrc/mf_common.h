@@ -169,9 +169,11 @@ __device__ __forceinline__ u32x4 ld_u32x4(const void* p) {
 
 // Bytes of a forward pass (inputs and output) from which its reads are streamed:
 // the inputs of a smaller one are still cached from the kernel that made them.
-// Prologue right after its producer, cached and streamed: 50 MB 13.3 and 14.4
-// us, 201 MB 39.6 and 36.2; conv, 269 MB, 47.9 and 43.2.
-constexpr size_t kStreamBytes = (size_t)128 << 20;
+// us, cached and streamed.  Prologue right after its producer: 50 MB 13.3 and
+// 14.4, 201 MB (192 MiB) 39.6 and 36.2.  Conv behind the producer of one input
+// and with a consumer: 128 MiB 49.4 and 53.7, 192 MiB 80.1 and 75.7, 256 MiB
+// 105.9 and 89.7, 512 MiB 203.9 and 191.4.
+constexpr size_t kStreamBytes = (size_t)192 << 20;
 
 // The same of a backward pass, whose gradient has just been made and whose
 // results are read next: about what the last-level cache holds (256 MB).

@@ -40,8 +40,8 @@ constexpr int kConvTile = 32;  // output tokens per thread
 // STREAM: read as a stream (bf16 only: fp32 touches a line with two loads of
 // 16 bytes per lane, and streamed it is slower, 46 -> 52 us forward and
 // 102 -> 127 backward at 4 x 4096 tokens of 768 channels, K = 4).  The forward,
-// which re-reads K - 1 rows in kConvTile, streams from kStreamBytes on and takes 55.7 -> 48.5 us at 8 x 4096 x
-// 1024 bf16 (50.9 -> 48.1 on another card).
+// which re-reads K - 1 rows in kConvTile, streams from kStreamBytes on and takes
+// 55.7 -> 48.5 us at 8 x 4096 x 1024 bf16 (50.9 -> 48.1 on another card).
 template <typename T, bool STREAM>
 struct Raw8 {
   bf16x8 v;
@@ -207,10 +207,11 @@ __global__ __launch_bounds__(256) void segmented_conv_kernel(ConvArgs a) {
           x0[e] = a.c ? cu[e] * acc[e] : acc[e];
           x1[e] = a.c ? cu[4 + e] * acc[4 + e] : acc[4 + e];
         }
-        // as streams: 46.1 -> 43.2 us at 4 x 4096 x 768 (the bf16 stores gain
-        // nothing: 50.9 and 51.9 at 8 x 4096 x 1024)
-        st_stream(reinterpret_cast<float*>(a.out) + off, x0);
-        st_stream(reinterpret_cast<float*>(a.out) + off + 4, x1);
+        // (plain stores: as streams the kernel alone takes 43.2 us against 46.1 at
+        // 4 x 4096 x 768, but with a consumer of the output behind it 83.3 against
+        // 78.0; the bf16 stores 50.9 and 51.9 at 8 x 4096 x 1024)
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + off) = x0;
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + off + 4) = x1;
       }
     }
   }

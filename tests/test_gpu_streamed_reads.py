@@ -1,4 +1,4 @@
-"""Forward passes of 128 MiB and more read their rows as streams: the bits of the smaller calls."""
+"""Forward passes of 192 MiB and more read their rows as streams: the bits of the smaller calls."""
 
 import pytest
 import torch
@@ -8,7 +8,7 @@ from mfattn.kernels import convolution, prologue
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", [5, 6])  # 126 MB and 151 MB; 126 MB is below the line
+@pytest.mark.parametrize("rows", [5, 6, 7, 8])  # 24 MiB a row: eight are at the line
 def test_prologue_rows_equal_rows_alone(rows, device):
     gen = torch.Generator(device=device).manual_seed(rows)
     q, k = (torch.randn((rows, 4096, h, 64), generator=gen, device=device).bfloat16() for h in (16, 8))
@@ -21,9 +21,9 @@ def test_prologue_rows_equal_rows_alone(rows, device):
 
 
 @pytest.mark.parametrize("taps", [1, 3, 8])
-@pytest.mark.parametrize("tokens", [4095, 4129])
+@pytest.mark.parametrize("tokens", [4095, 4129, 6143, 6145])
 def test_conv_rows_equal_rows_alone(taps, tokens, device):
-    """Four rows of 1024 channels are 134 MB either side of 2**27 bytes."""
+    """Four rows of 1024 channels in four tensors are either side of 192 MiB at 6144 tokens."""
     gen = torch.Generator(device=device).manual_seed(taps)
     b, c, v = (torch.randn((4, tokens, 1024), generator=gen, device=device).bfloat16() for _ in range(3))
     w = torch.randn((1024, taps), generator=gen, device=device).bfloat16()
