@@ -433,11 +433,10 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
 // dQ^T += K^T dS^T takes its K^T operand from the K tile through
 // transposing LDS reads.
 // ---------------------------------------------------------------------------
-template <int HPW>
-__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(HPW + 2)))
+template <int HPW, int SLOT>  // SLOT: 64-key stages per ring slot
+__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(HPW < SLOT ? 2 : HPW + 2)))
 void bwd_dq_bf16_kernel(BwdArgs a) {
   constexpr int W = 4 * HPW;
-  constexpr int SLOT = HPW;  // 64-key stages per ring slot
   __shared__ __attribute__((aligned(16))) char slotA[SLOT * kStageBytes], slotB[SLOT * kStageBytes];
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
@@ -967,10 +966,8 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
   a.Hq = Hq;
   a.Hkv = Hkv;
   a.G = Hq / Hkv;
-  // dq: two heads per workgroup where the group splits into pairs; one, with
-  // one-stage ring slots (three workgroups per CU at 132 VGPRs), for odd
-  // groups (8 x 4096, segments 32-2048, 12/4 heads: 156 us against 170 with
-  // two-stage slots, 8/8: 104 against 112).  Small even calls keep two heads:
+  // dq: two heads per workgroup where the group splits into pairs, one for odd
+  // groups (one_stage_slots has their slots).  Small even calls keep two heads:
   // one measured 24 us against 20.5 at 1 x 8192 of short segments and -6 to
   // +5% at others.
   const int hpw = (a.G % 2 == 0) ? 2 : 1;
@@ -1013,9 +1010,11 @@ hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const vo
                });
   } else {
     if (hpw == 2)
-      hipLaunchKernelGGL((bwd_dq_bf16_kernel<2>), qgrid, dim3(512), 0, stream, a);
+      hipLaunchKernelGGL((bwd_dq_bf16_kernel<2, 2>), qgrid, dim3(512), 0, stream, a);
+    else if (one_stage_slots(mode, a.nq, qgrid.x))
+      hipLaunchKernelGGL((bwd_dq_bf16_kernel<1, 1>), qgrid, dim3(256), 0, stream, a);
     else
-      hipLaunchKernelGGL((bwd_dq_bf16_kernel<1>), qgrid, dim3(256), 0, stream, a);
+      hipLaunchKernelGGL((bwd_dq_bf16_kernel<1, 2>), qgrid, dim3(256), 0, stream, a);
   }
   const dim3 kgrid(Hkv * batch * lay.nk);
   if (phases & 4) {

@@ -231,10 +231,11 @@ void attn_fwd_f32_kernel(FwdArgs a) {
 // (1, 1), a full-rate VALU op that halves the adds.
 //
 // A workgroup serves HPW heads, four waves each.  Two heads share every K/V
-// stage and win where the chip is full.  One head takes ring slots of one
+// stage and win where the chip is full.  One head with ring slots of one
 // stage (33 KB of LDS, so four workgroups fit a CU, as two two-head ones do)
-// and is the finer unit; a wave's arithmetic, and so every output bit, is the
-// same.  heads_per_block has the rule and what both measure.
+// is the finer unit; a wave's arithmetic, and so every output bit, is the
+// same.  heads_per_block and one_stage_slots have the rules and what they
+// measure.
 // ---------------------------------------------------------------------------
 // The query half of the attention prologue on the query fragments a lane
 // holds (dims 16 ks + 8 half .. +7 of one query row, ks = 0..3; the other
@@ -316,11 +317,10 @@ __device__ __forceinline__ void rope_query(const FwdArgs& a, int b, int qpos, in
   }
 }
 
-template <int HPW, bool ROPE>
-__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(4)))
+template <int HPW, int SLOT, bool ROPE>  // SLOT: 64-key stages per ring slot
+__global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(HPW < SLOT ? 2 : 4)))
 void attn_fwd_bf16_kernel(FwdArgs a) {
   constexpr int W = 4 * HPW;
-  constexpr int SLOT = HPW;  // 64-key stages per ring slot
   __shared__ __attribute__((aligned(16))) char slotA[SLOT * kStageBytes], slotB[SLOT * kStageBytes];
   const int lane = threadIdx.x & 63;
   // scalar wave index: keeps the DMA destinations scalar expressions of the
@@ -500,9 +500,9 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
     if (run[1]) finish_pv(s1, vt, 1);
   };
 
-  // Ring of two slots (two 64-key stages each with two heads, one with one):
-  // the DMAs of slot i+1 are issued right after the barrier that opens slot i,
-  // so they have the compute of slot i to land, and one barrier serves a slot.
+  // Ring of two slots: the DMAs of slot i+1 are issued right after the barrier
+  // that opens slot i, so they have the compute of slot i to land, and one
+  // barrier serves a slot.
   auto issue_slot = [&](int i, int e0, int e1, char* slot) {
     if (SLOT * i < nsteps) issue(e0, slot);
     if (SLOT == 2 && 2 * i + 1 < nsteps) issue(e1, slot + kStageBytes);
@@ -561,8 +561,7 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
 
 // Heads per workgroup of the bf16 forward: one for odd groups and for calls
 // whose one-head workgroups are all resident at once (four on each of the 256
-// CUs), two otherwise.  us with two heads (odd groups: one head with two-stage
-// slots, two workgroups per CU) and with one:
+// CUs), two otherwise.  us with two heads and with one:
 //   1 x 5003, one causal segment, 16/8 heads   128 -> 110    (640 workgroups)
 //   1 x 2048, mean segment 512, 16/8            19.2 -> 15.9 (256)
 //   1 x 8192, one segment, 16/8                217 -> 200    (1024)
@@ -570,8 +569,6 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
 //   1 x 16384, segments 16-128, 16/8            31.5 -> 32.0 (2048: two)
 //   4 x 8192, mean segment 512, 16/8            98 -> 106    (4096: two)
 //   4 x 4096, mean segment 512, 32/8            75 -> 86     (4096: two)
-//   8 x 4096, segments 32-2048, 12/4           127 -> 104    (odd)
-//   8 x 4096, segments 32-2048, 8/8             85.5 -> 72   (odd)
 static int heads_per_block(int G, long long tile_heads) {
   return G % 2 == 0 && tile_heads > 4 * 256 ? 2 : 1;
 }
@@ -617,6 +614,16 @@ static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, 
   return a;
 }
 
+template <bool ROPE>
+static void launch_fwd_bf16(const FwdArgs& a, int hpw, int mode, dim3 grid, hipStream_t stream) {
+  if (hpw == 2)
+    hipLaunchKernelGGL((attn_fwd_bf16_kernel<2, 2, ROPE>), grid, dim3(512), 0, stream, a);
+  else if (a.G % 2 == 0 || one_stage_slots(mode, a.nq, grid.x))
+    hipLaunchKernelGGL((attn_fwd_bf16_kernel<1, 1, ROPE>), grid, dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((attn_fwd_bf16_kernel<1, 2, ROPE>), grid, dim3(256), 0, stream, a);
+}
+
 hipError_t launch_attn_fwd(const void* q, const void* k, const void* v, bool f32, int batch,
                            int T, int S, int Hq, int Hkv, int mode, float scale,
                            const void* plan, void* out, float* lse, hipStream_t stream) {
@@ -630,10 +637,7 @@ hipError_t launch_attn_fwd(const void* q, const void* k, const void* v, bool f32
                  hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(blocks), dim3(256), 0, stream, a);
                });
   } else {
-    if (hpw == 2)
-      hipLaunchKernelGGL((attn_fwd_bf16_kernel<2, false>), grid, dim3(512), 0, stream, a);
-    else
-      hipLaunchKernelGGL((attn_fwd_bf16_kernel<1, false>), grid, dim3(256), 0, stream, a);
+    launch_fwd_bf16<false>(a, hpw, mode, grid, stream);
   }
   return hipGetLastError();
 }
@@ -676,10 +680,7 @@ hipError_t launch_attn_fwd_rope_q(const void* q_raw, const void* k, const void* 
   hipLaunchKernelGGL(rope_table_kernel, dim3((unsigned)((tokens * (kD / 2) + 255) / 256)),
                      dim3(256), 0, stream, a, reinterpret_cast<uint32_t*>(table), tokens);
   const dim3 grid(Hkv * a.hchunks * batch * a.nq);
-  if (hpw == 2)
-    hipLaunchKernelGGL((attn_fwd_bf16_kernel<2, true>), grid, dim3(512), 0, stream, a);
-  else
-    hipLaunchKernelGGL((attn_fwd_bf16_kernel<1, true>), grid, dim3(256), 0, stream, a);
+  launch_fwd_bf16<true>(a, hpw, mode, grid, stream);
   return hipGetLastError();
 }
 

@@ -40,6 +40,35 @@
 
 namespace mf {
 
+// Whether the one-head workgroups (odd groups) of the bf16 forward and dq take
+// ring slots of one 64-key stage (33 KB of LDS: four workgroups per CU in the
+// forward, three in dq) instead of two (66 KB: two per CU, half the barriers).
+// Up to two workgroups per CU both forms are resident whole and two stages are
+// equal or up to 4 % faster.  With more, one stage hides more latency, but until
+// there are clearly more than it keeps resident at once (1024), unequal lists
+// stay on the CU they were dealt to; only key-mask rows, whose lists are equal,
+// and rows of up to four tiles, whose lists are short, gain there throughout.
+// us, two stages -> one, forward / dq:
+//   3/1,   192 workgroups, 1 x 8192 causal, one segment    116 -> 118, 133 -> 138
+//   8/8,   512,  the same                                  139 -> 138, 161 -> 166
+//   24/8,  768,  1 x 4096 causal, one segment             72.2 -> 77.5, 87.8 -> 93.0
+//   24/8,  768,  the same, segments 16-128                17.5 -> 14.5, 21.6 -> 17.5
+//   12/4,  768,  1 x 8192 bidirectional, segments 64-1024 46.2 -> 46.1, 49.3 -> 53.3
+//   12/4,  720,  20 x 333 padded                          25.2 -> 19.2, 27.5 -> 23.0
+//   12/4,  768,  64 x 128 bidirectional                   15.4 -> 11.9, 18.6 -> 15.4
+//   12/4,  768,  16 x 500 causal, one segment             19.0 -> 18.0, 23.6 -> 21.9
+//   8/8,   800,  1 x 12800 causal, segments 64-1024       28.2 -> 29.8, 30.9 -> 33.5
+//   24/8, 1128,  1 x 6000 causal, one segment              158 -> 168, 186 -> 200
+//   12/4, 1536,  1 x 16384 causal, one segment             561 -> 523, 693 -> 665
+//   24/8, 1536,  1 x 8192, one segment                     280 -> 264, 329 -> 341
+//   24/8, 1536,  1 x 8192, segments 64-1024               45.7 -> 37.3, 52.8 -> 46.6
+//   8/8,  2048,  4 x 8192 causal, one segment              334 -> 344, 408 -> 415
+//   8/8,  2048,  8 x 4096 bidirectional, 32-2048           130 -> 107, 149 -> 133
+//   12/4, 3072,  the same                                  193 -> 167, 225 -> 203
+inline bool one_stage_slots(int mode, int row_tiles, long long workgroups) {
+  return workgroups > (mode == 2 || row_tiles <= 4 ? 2 * 256 : 5 * 256);
+}
+
 constexpr int kRowBytes = 128;
 constexpr int kTileBytes = 64 * kRowBytes;
 
