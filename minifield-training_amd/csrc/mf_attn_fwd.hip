@@ -559,18 +559,35 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
   }
 }
 
-// Heads per workgroup of the bf16 forward: one for odd groups and for calls
-// whose one-head workgroups are all resident at once (four on each of the 256
-// CUs), two otherwise.  us with two heads and with one:
-//   1 x 5003, one causal segment, 16/8 heads   128 -> 110    (640 workgroups)
-//   1 x 2048, mean segment 512, 16/8            19.2 -> 15.9 (256)
-//   1 x 8192, one segment, 16/8                217 -> 200    (1024)
-//   1 x 8192, segments 16-128, 16/8             17.6 -> 18.5 (1024)
-//   1 x 16384, segments 16-128, 16/8            31.5 -> 32.0 (2048: two)
-//   4 x 8192, mean segment 512, 16/8            98 -> 106    (4096: two)
-//   4 x 4096, mean segment 512, 32/8            75 -> 86     (4096: two)
-static int heads_per_block(int G, long long tile_heads) {
-  return G % 2 == 0 && tile_heads > 4 * 256 ? 2 : 1;
+// Heads per workgroup of the bf16 forward, even groups (odd ones take one, see
+// one_stage_slots): two share every K/V stage; one is the finer unit, and with
+// slots of one stage four fit a CU.  What decides is the heads the fullest CU
+// gets, ceil(w / 256) of w tile-heads against 2 ceil(w / 512).  They differ up to
+// 256 and from 513 to 768, where one head wins.  From 257 to 512 they are equal:
+// one still wins for causal rows of several tiles, whose lists differ in length,
+// elsewhere it wins or loses with the lists.  Beyond 768 it does too, and two
+// heads are taken; so are they from 257 on for rows of one tile.  us with two heads
+// and with one:
+//   1 x 2048 causal, segments 128-1024, 16/8  (w = 256)     26.9 -> 22.1
+//   1 x 2048 bidirectional, one segment, 16/8 (256)         41.7 -> 34.2
+//   1 x 4096 causal, one segment, 16/8        (512)         77.1 -> 65.9
+//   1 x 4096 causal, segments 16-128, 16/8    (512)         11.6 -> 10.7
+//   1 x 4096 bidirectional, one segment, 16/8 (512)         82.0 -> 86.2 (two)
+//   1 x 4096 bidirectional, 64-1024, 16/8     (512)         48.4 -> 40.4 (two)
+//   32 x 128, one segment, 16/8               (512)          8.1 -> 8.3  (two)
+//   1 x 5003 causal, one segment, 16/8        (640)          122 -> 102
+//   1 x 6000 bidirectional, one segment, 16/8 (752)          219 -> 197
+//   6 x 1000 causal, segments 16-128, 16/8    (768)         16.3 -> 14.1
+//   48 x 128 causal, one segment, 16/8        (768)         11.7 -> 12.3 (two)
+//   1 x 7168 causal, one segment, 16/8        (896)          143 -> 151  (two)
+//   1 x 8192 causal, one segment, 16/8        (1024)         213 -> 197  (two)
+//   4 x 2048 causal, segments 16-128, 16/8    (1024)        16.9 -> 17.7 (two)
+//   1 x 4096 bidirectional, one segment, 32/8 (1024)         147 -> 157  (two)
+//   4 x 8192, mean segment 512, 16/8          (4096)          98 -> 106  (two)
+static int heads_per_block(int G, int mode, int nq, long long tile_heads) {
+  if (G % 2 || tile_heads <= 256) return 1;
+  if (nq == 1 || tile_heads > 3 * 256) return 2;
+  return mode == 0 || tile_heads > 2 * 256 ? 1 : 2;
 }
 
 // Arguments of one forward launch: operands, the plan's sections, shapes and
@@ -596,7 +613,7 @@ static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, 
   a.Hq = Hq;
   a.Hkv = Hkv;
   a.G = Hq / Hkv;
-  *hpw = heads_per_block(a.G, (long long)batch * lay.nq * Hq);
+  *hpw = heads_per_block(a.G, mode, lay.nq, (long long)batch * lay.nq * Hq);
   a.hchunks = a.G / *hpw;
   a.nq = lay.nq;
   a.nk = lay.nk;
