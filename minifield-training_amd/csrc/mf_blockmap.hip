@@ -47,20 +47,28 @@ __device__ __forceinline__ int packed_id(const MapArgs& a, int b, int p) {
   return active ? s : 0;
 }
 
-// Key-mask mode: whether row b has an active key (bidirectional.py:23), for a
-// whole wave.  512 keys a round, until one is active: the first round in all
-// but rows that open with padding.
-__device__ __forceinline__ bool row_has_key(const MapArgs& a, int b) {
+// Whether any of the keys base .. base + 64 * N - 1 of row b is active (keys past
+// the row re-read its last one), for a whole wave.
+template <int N>
+__device__ __forceinline__ bool any_key(const MapArgs& a, int b, int base) {
   const int lane = threadIdx.x & 63;
-  for (int base = 0; base < a.kv_len; base += 512) {
-    int any = 0;
+  int any = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int p = min(base + 64 * i + lane, a.kv_len - 1);
-      any |= mask_at(a.mask, a.mask_u8, (long)b * a.kv_len + p);
-    }
-    if (__any(any != 0)) return true;
+  for (int i = 0; i < N; ++i) {
+    const int p = min(base + 64 * i + lane, a.kv_len - 1);
+    any |= mask_at(a.mask, a.mask_u8, (long)b * a.kv_len + p);
   }
+  return __any(any != 0);
+}
+
+// Key-mask mode: whether row b has an active key (bidirectional.py:23), for a
+// whole wave.  The first 512 keys answer for all but rows that open with padding;
+// those are read on in rounds of 2048, whose loads are in flight together (map of
+// one left-padded row of 32768 keys: 33 us in rounds of 512, 29 with 2048).
+__device__ __forceinline__ bool row_has_key(const MapArgs& a, int b) {
+  if (any_key<8>(a, b, 0)) return true;
+  for (int base = 512; base < a.kv_len; base += 2048)
+    if (any_key<32>(a, b, base)) return true;
   return false;
 }
 
@@ -387,9 +395,11 @@ __global__ __launch_bounds__(256) void placement_ids_kernel(MapArgs a, const int
 // The same order for up to kRankItems items a side, one per thread: an item's
 // place is its bucket's start, plus the bucket's items in earlier waves, plus
 // those in earlier lanes (the lanes of a bucket from one ballot per bucket
-// bit).  2.2 us for 72 items between idle neighbours, where the counting sort
-// above, whose threads take several items and scan the buckets serially, takes
-// 3.2; behind a busy kernel a launch of this size costs 4.6 us either way.
+// bit).  The counting sort above, whose threads take several items and scan the
+// buckets serially, makes the map 1.0 to 1.9 us longer: map and forward in one
+// chain 20.2 -> 18.9 us at 2 x 256, 25.1 -> 23.6 at 1 x 2048, 64.9 -> 63.2 at 1 x
+// 32768 of short segments (each less noisy than that), 39.3 -> 39.0 at 24 x 333
+// and nothing measurable from 8 x 4096 on.
 constexpr int kRankItems = 1024;
 
 __global__ __launch_bounds__(kRankItems) void order_rank_kernel(MapArgs a) {

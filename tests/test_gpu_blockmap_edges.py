@@ -18,7 +18,7 @@ def test_order_item_counts(rows, t, device):
     _check(0, mask, seg, t, t, device)
 
 
-@pytest.mark.parametrize("s", [1, 511, 512, 513, 1300])
+@pytest.mark.parametrize("s", [1, 511, 512, 513, 1300, 2560, 2561, 4700])
 def test_key_mask_rows_with_late_or_no_keys(s, device):
     rng = np.random.default_rng(s)
     mask = np.zeros((6, s), np.int32)
