@@ -36,8 +36,14 @@ def test_reference_cached_fixture(device):
     (torch.bfloat16, 8, 2),   # 4 query heads per KV head
     (torch.bfloat16, 2, 2),   # 1
     (torch.bfloat16, 4, 2),   # 2
-    (torch.bfloat16, 6, 2),   # 3: served by the LDS-staged kernel
+    (torch.bfloat16, 6, 2),   # 3: the row kernel with fp32 probabilities
     (torch.bfloat16, 16, 2),  # 8
+    (torch.bfloat16, 12, 1),  # 12: the LDS-staged kernel, one pass of 8 heads and one of 4
+    (torch.bfloat16, 9, 3),   # 3 over three KV heads: the LDS-staged kernel, one pass of 3
+    (torch.bfloat16, 3, 3),   # three KV heads and groups of 1, 2, 4 and 8: decode_bf16_kernel
+    (torch.bfloat16, 6, 3),
+    (torch.bfloat16, 12, 3),
+    (torch.bfloat16, 24, 3),
     (torch.bfloat16, 32, 2),  # 16: the LDS-staged kernel in two passes of 8 heads
     (torch.float32, 24, 2),   # 12: one pass of 8 heads and one of 4
     (torch.bfloat16, 40, 1),  # 40: five passes, one KV head
@@ -98,11 +104,18 @@ def test_scalar_length_broadcasts_and_backends_agree(device):
 
 @pytest.mark.parametrize("dtype,hq,hkv", [
     (torch.float32, 8, 2),
-    (torch.bfloat16, 8, 2),   # the streaming kernel appends (G = 4)
+    (torch.bfloat16, 8, 2),   # the row kernel appends (G = 4)
     (torch.bfloat16, 2, 2),   # G = 1
     (torch.bfloat16, 16, 2),  # G = 8
-    (torch.bfloat16, 6, 2),   # G = 3: the prep kernel appends, the LDS-staged kernel decodes
-    (torch.bfloat16, 32, 2),  # G = 16: likewise, in two passes of 8 query heads
+    (torch.bfloat16, 6, 2),   # G = 3
+    (torch.bfloat16, 32, 2),  # G = 16: the prep kernel appends, the LDS-staged kernel decodes in
+                              # two passes of 8 query heads
+    (torch.bfloat16, 12, 1),  # G = 12: likewise, passes of 8 and 4
+    (torch.bfloat16, 9, 3),   # G = 3 over three KV heads: likewise, one pass of 3
+    (torch.bfloat16, 3, 3),   # three KV heads and groups of 1, 2, 4 and 8: decode_bf16_kernel
+    (torch.bfloat16, 6, 3),
+    (torch.bfloat16, 12, 3),
+    (torch.bfloat16, 24, 3),
 ])
 def test_decode_step_appends_per_row(dtype, hq, hkv, device):
     """Ragged KV-cache append + decode (layers/attention.py:309-317, one slot per row).

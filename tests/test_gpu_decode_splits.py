@@ -12,9 +12,10 @@ pytestmark = pytest.mark.gpu
 
 
 # rows x ceil(capacity / 128) items: up to 256 the most waves an item, up to 512 four, then one;
-# caches above 256 MiB stream V
+# up to 128 slots an item of several waves writes the output itself
 @pytest.mark.parametrize("rows, cap", [(3, 127), (3, 128), (3, 129), (128, 200), (129, 200),
-                                       (256, 130), (257, 130)])
+                                       (256, 130), (257, 130), (256, 128), (300, 128), (300, 100),
+                                       (512, 64), (513, 64)])
 @pytest.mark.parametrize("hq, hkv", [(8, 8), (16, 8), (40, 8), (64, 8), (12, 4), (10, 2), (7, 1),
                                      (8, 1)])
 def test_splits_against_fp64(rows, cap, hq, hkv, device):
@@ -44,3 +45,30 @@ def test_splits_against_fp64(rows, cap, hq, hkv, device):
     k[at, pos.long()], v[at, pos.long()] = kn[:, 0], vn[:, 0]
     assert torch.equal(kc, k) and torch.equal(vc, v)
     assert torch.equal(step, attention.dense_cached_attention(q, k, v, pos + 1))
+
+
+@pytest.mark.parametrize("group", [1, 2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("hkv, rows, cap", [(8, 520, 260), (4, 520, 520), (2, 1030, 520),
+                                            (1, 1030, 1024)])
+def test_caches_that_stream_v(hkv, rows, cap, group, device):
+    """K and V of 264 to 277 MiB, above the 256 MiB from which V streams too, one wave an item:
+    a plain decode against float64 on some rows, and a step with an append (the decode of the
+    written cache, bit for bit)."""
+    assert rows * cap * hkv * 64 * 4 > 256 << 20
+    hq = hkv * group
+    gen = torch.Generator(device=device).manual_seed(hq + cap)
+    mk = lambda *s: torch.randn(s, generator=gen, device=device).bfloat16()  # noqa: E731
+    q, kn, vn = mk(rows, 1, hq, 64), mk(rows, 1, hkv, 64), mk(rows, 1, hkv, 64)
+    k, v = mk(rows, cap, hkv, 64), mk(rows, cap, hkv, 64)
+    lengths = torch.randint(1, cap + 1, (rows,), generator=gen, device=device, dtype=torch.int32)
+    lengths[:4] = torch.tensor([cap, 0, 1, 129], dtype=torch.int32)
+    out = attention.dense_cached_attention(q, k, v, lengths)
+    some = [0, 1, 2, 3, 7, rows // 2, rows - 1]
+    ref = oatt.cached_fp64(*(x[some].float().cpu().numpy() for x in (q, k, v)),
+                           lengths[some].cpu().numpy())[0]
+    check_bf16(f"decode streamed {hq}/{hkv}", out[some], ref)
+    pos = (lengths - 1).clamp(min=0)
+    step, kc, vc = attention.cached_attention_step(q, kn, vn, k, v, pos, backend="hip")
+    at = torch.arange(rows, device=device)
+    assert torch.equal(kc[at, pos.long()], kn[:, 0]) and torch.equal(vc[at, pos.long()], vn[:, 0])
+    assert torch.equal(step, attention.dense_cached_attention(q, kc, vc, pos + 1))
