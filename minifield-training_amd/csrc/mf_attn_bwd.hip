@@ -84,11 +84,13 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(BwdArgs a, int B) {
     const float* o = reinterpret_cast<const float*>(a.out) + idx * kD;
     const float* g = reinterpret_cast<const float*>(a.dout) + idx * kD;
 #pragma unroll
-    for (int c4 = 0; c4 < 16; ++c4) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(o + c4 * 4);
-      const f32x4 y = *reinterpret_cast<const f32x4*>(g + c4 * 4);
+    for (int c4 = 0; c4 < 8; ++c4) {  // dims d and 32 + d in turn, as dq adds them
+      const f32x4 x0 = *reinterpret_cast<const f32x4*>(o + c4 * 4);
+      const f32x4 x1 = *reinterpret_cast<const f32x4*>(o + 32 + c4 * 4);
+      const f32x4 y0 = *reinterpret_cast<const f32x4*>(g + c4 * 4);
+      const f32x4 y1 = *reinterpret_cast<const f32x4*>(g + 32 + c4 * 4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = fmaf(x[e], y[e], acc);
+      for (int e = 0; e < 4; ++e) acc = fmaf(x1[e], y1[e], fmaf(x0[e], y0[e], acc));
     }
   }
   const size_t li = ((size_t)b * a.Hq + h) * a.T + t;
@@ -141,14 +143,19 @@ void bwd_dq_f32_kernel(BwdArgs a) {
   if (a.fuse_delta) {
     f32_store(kt[wave], lane, kx);  // O
     wave_lds_fence();
+    // D in the order in which the MFMA steps add dP's products (dims d and 32 + d
+    // in turn), from zero as dP: where P is near 1 the two cancel, and so then do
+    // their rounding errors (dq of one-token segments, whose gradient is zero,
+    // was off by 1e-6 with D in another order or dP started from -D, 1e-7 so)
     float part = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const f32x4 ox = kt[wave].row4(lane, j);
+      const f32x4 o0 = kt[wave].row4(col, j), o1 = kt[wave].row4(col + 32, j);
+      const f32x4 g0 = vt[wave].row4(col, j), g1 = vt[wave].row4(col + 32, j);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) part = fmaf(ox[e], gf[j][e], part);
+      for (int e = 0; e < 4; ++e) part = fmaf(o1[e], g1[e], fmaf(o0[e], g0[e], part));
     }
-    nd = -halves_sum(part);
+    nd = -part;
   } else {
     nd = a.ndelta[li];
   }
@@ -205,9 +212,7 @@ void bwd_dq_f32_kernel(BwdArgs a) {
     f32_store(vt[wave], lane, vx, a.S - kb);
     wave_lds_fence();
     more = fetch(i);
-    f32x16 s = zero16(), dp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dp[r] = nd;
+    f32x16 s = zero16(), dp = zero16();
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const f32x4 kr = kt[wave].row4(lane, j), qr = qt.row4(lane, j);
@@ -232,7 +237,7 @@ void bwd_dq_f32_kernel(BwdArgs a) {
       for (int r = 0; r < 16; ++r) s[r] = kb + acc_row(r, lane) <= qpos ? s[r] : kNegInf;
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(fmaf(s[r], c, -lse2)) * dp[r];
+    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(fmaf(s[r], c, -lse2)) * (dp[r] + nd);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       dqacc[0] = mfma32x32x2(kt[wave].col(lane, 0, r), s[r], dqacc[0]);
@@ -352,16 +357,10 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
     f32_store(gt[wave], lane, gx, a.T - qb);
     wave_lds_fence();
     it = fetch(it + kKvWaves);
-    f32x16 s = zero16(), dp;
+    f32x16 s = zero16(), dp = zero16();
     auto row4 = [&](int which, int g4) {
       return *reinterpret_cast<const f32x4*>(&rows[wave][which][8 * g4 + 4 * half]);
     };
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const f32x4 d4 = row4(1, g4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dp[g4 * 4 + e] = d4[e];
-    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const f32x4 kr = kt.row4(lane, j), qr = qt[wave].row4(lane, j);
@@ -387,12 +386,12 @@ void bwd_dkdv_f32_kernel(BwdArgs a) {
     }
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
-      const f32x4 l4 = row4(0, g4);
+      const f32x4 l4 = row4(0, g4), d4 = row4(1, g4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int r = g4 * 4 + e;
         s[r] = fast_exp2(fmaf(s[r], c, -l4[e]));
-        dp[r] *= s[r];
+        dp[r] = (dp[r] + d4[e]) * s[r];
       }
     }
 #pragma unroll

@@ -50,3 +50,26 @@ def test_more_workgroups_than_one_launch_may_have(device):
     assert torch.allclose(dv, do.view(rows, 1, hkv, 2, 64).sum(3), rtol=1e-5, atol=2e-5)
     # dS = P (dP - D): dP and D are the same 64 products in another order
     assert dq.abs().max() < 1e-4 and dk.abs().max() < 1e-4
+
+
+def test_one_token_segments_have_gradients_of_the_rounding_alone(device):
+    """A token that sees only itself has P = 1 and O = V, so dP - D is zero but for the roundings
+    of O, two per dimension: their root mean square is at most 2**-24 sqrt(2) times the 2-norm of
+    the 64 products of dO and V, as long as the sums of dP and D round alike.  (Sums in different
+    orders, or dP started from -D, add sqrt(64) roundings of partial sums: several times that.)"""
+    gen = torch.Generator(device=device).manual_seed(5)
+    rows, t, h = 4, 100, 8
+    q, k, v, do = (torch.randn((rows, t, h, 64), generator=gen, device=device) for _ in range(4))
+    seg = torch.arange(1, t + 1, device=device, dtype=torch.int32).repeat(rows, 1)
+    plan = ops.block_map(seg, seg, 0, t, t)
+    out, lse = ops.attn_fwd(q, k, v, plan, 0, 0.125)
+    dq, dk, _ = ops.attn_bwd(q, k, v, out, do, lse, plan, 0, 0.125)
+    ws = ops.bwd_workspace(q)
+    ops.attn_bwd_delta(out, do, lse, ws)
+    dq2 = torch.empty_like(q)
+    ops.attn_bwd_dq(q, k, v, do, lse, plan, 0, 0.125, ws, dq2)
+    assert torch.equal(dq, dq2)  # the separate pass adds D in the same order
+    rms = lambda x: x.double().square().mean().sqrt().item()  # noqa: E731
+    products = (do.double() * v.double()).square().sum(-1).mean().sqrt().item()
+    bound = 2.0 ** -24 * 2 ** 0.5 * products * 0.125
+    assert rms(dq) <= bound * rms(k) and rms(dk) <= bound * rms(q)
