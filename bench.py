@@ -486,20 +486,20 @@ TRAFFIC_KERNELS = {
     # bench name -> (device kernels as name prefixes, workload, which dispatch of each kernel:
     # None = the mean over the run's dispatches; 0 / 1 = the first / second, for kernels that
     # --profile-step launches for two different calls)
-    "block_map": (("mf::token_ids_kernel", "mf::tile_runs_kernel", "mf::tile_lists_kernel",
+    "block_map": (("mf::tile_runs_kernel", "mf::tile_lists_kernel", "mf::order_rank_kernel",
                    "mf::order_kernel"), "C2", None),
-    # the plain forward only (the instances with the query prologue are <., true>)
-    "attn_fwd": (("mf::attn_fwd_bf16_kernel<2, false>", "mf::attn_fwd_bf16_kernel<1, false>"),
-                 "C2", None),
+    # the plain forward only (the instances with the query prologue are <., ., true>)
+    "attn_fwd": (("mf::attn_fwd_bf16_kernel<2, 2, false>", "mf::attn_fwd_bf16_kernel<1, 1, false>",
+                  "mf::attn_fwd_bf16_kernel<1, 2, false>"), "C2", None),
     "attn_bwd_dq": (("mf::bwd_dq_bf16_kernel<",), "C2", None),  # computes D itself in the product call
     "attn_bwd_dkdv": (("mf::bwd_dkdv_bf16_kernel",), "C2", None),
     "decode": (("mf::decode_prep_kernel", "mf::decode_rows_kernel<", "mf::decode_bf16_kernel<",
                 "mf::decode_combine_kernel<"), "C4", 0),
     "decode_append": (("mf::decode_rows_kernel<", "mf::decode_bf16_kernel<",
                        "mf::decode_combine_kernel<"), "C4", 1),
-    # the first dispatch: the qk_norm_rope row (the composite rows after it launch it again,
-    # the last one for the keys alone)
-    "qk_norm_rope": (("mf::qk_norm_rope_kernel<",), "C2", 0),
+    # the first dispatch of the streaming form: the qk_norm_rope row (the composite rows after it
+    # launch it again; the keys alone take the other form)
+    "qk_norm_rope": (("mf::qk_norm_rope_kernel<false, true>",), "C2", 0),
     "qk_norm_rope_bwd": (("mf::qk_norm_rope_bwd_kernel<", "mf::rope_gain_reduce_kernel"), "C2",
                          None),
     "segmented_conv": (("mf::segmented_conv_kernel<",), "C2", None),

@@ -128,9 +128,9 @@ __device__ __forceinline__ bf16x4 scaled_bf16x4(const f32x16& v, int base, float
 }
 
 // Writes a wave's transposed 32 x 64 accumulator tile (lane = row `lane & 31`,
-// acc[db][4 g + i] = dim 32 db + 8 g + 4 half + i) as bf16 rows `stride`
-// elements apart, scaled or zeroed as scaled_bf16x4; `row` is the lane's own
-// row.  All 64 lanes of a written row pair (l, l ^ 32) take part.
+// acc[db][4 g + i] = dim 32 db + 8 g + 4 half + i) as bf16 rows, scaled or
+// zeroed as scaled_bf16x4; `row` is the lane's own row.  Both lanes of a written
+// row (l, l ^ 32) take part.
 //
 // What bounds the store is the number of L2 write requests, not the bytes: as
 // accumulated, a lane holds four neighbouring dims, and an 8-byte store per

@@ -920,7 +920,10 @@ constexpr long long kMostWavesItems = 256;
 constexpr long long kFourWavesItems = 512;
 // Caches (K and V, all rows) that fit the 256 MB last-level cache keep V
 // cacheable, larger ones stream: 16 x 8192 takes 36.6 us so and 38.4 with both
-// streamed, 64 x 8192 114.0 and 111.1, 256 x 1024 69.1 and 65.3.
+// streamed, 64 x 8192 114.0 and 111.1, 256 x 1024 69.1 and 65.3.  That is with
+// other caches in between, as the layers of a model come; one cache of 64 x 8192
+// (half full) decoded over and over finds part of V still there, 109 and 117 us,
+// against 104 and 100 in turn with two others.
 constexpr long long kKeepBytes = 256ll << 20;
 
 hipError_t launch_decode(const void* q, const void* k, const void* v, const int32_t* lengths,
