@@ -563,11 +563,13 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
 // one_stage_slots): two share every K/V stage; one is the finer unit, and with
 // slots of one stage four fit a CU.  What decides is the heads the fullest CU
 // gets, ceil(w / 256) of w tile-heads against 2 ceil(w / 512).  They differ up to
-// 256 and from 513 to 768, where one head wins.  From 257 to 512 they are equal:
-// one still wins for causal rows of several tiles, whose lists differ in length,
-// elsewhere it wins or loses with the lists.  Beyond 768 it does too, and two
-// heads are taken; so are they from 257 on for rows of one tile.  us with two heads
-// and with one:
+// 256 and from 513 to 768, where one head wins.  Where they are equal, one head
+// still wins if the tiles' lists differ in length, and loses up to 8 % if they do
+// not: it is taken for causal rows of several tiles up to 512, and up to 1024 for
+// several rows of at least eight (one row alone keeps the order its own tiles
+// come in), where it loses at most 4 % on short segments.  Bidirectional calls
+// there, whose lists are equal when a row is one segment, and rows of one tile
+// keep two.  us with two heads and with one:
 //   1 x 2048 causal, segments 128-1024, 16/8  (w = 256)     26.9 -> 22.1
 //   1 x 2048 bidirectional, one segment, 16/8 (256)         41.7 -> 34.2
 //   1 x 4096 causal, one segment, 16/8        (512)         77.1 -> 65.9
@@ -579,14 +581,18 @@ void attn_fwd_bf16_kernel(FwdArgs a) {
 //   1 x 6000 bidirectional, one segment, 16/8 (752)          219 -> 197
 //   6 x 1000 causal, segments 16-128, 16/8    (768)         16.3 -> 14.1
 //   48 x 128 causal, one segment, 16/8        (768)         11.7 -> 12.3 (two)
-//   1 x 7168 causal, one segment, 16/8        (896)          143 -> 151  (two)
-//   1 x 8192 causal, one segment, 16/8        (1024)         213 -> 197  (two)
-//   4 x 2048 causal, segments 16-128, 16/8    (1024)        16.9 -> 17.7 (two)
+//   1 x 7168 causal, one segment, 16/8        (896)          148 -> 156  (two)
+//   1 x 7168 causal, segments 64-1024, 16/8   (896)         34.4 -> 29.7 (two)
+//   2 x 3400 causal, one segment, 16/8        (864)         94.6 -> 83.0
+//   4 x 2048 causal, one segment, 16/8        (1024)        55.3 -> 50.1
+//   4 x 2048 causal, segments 16-128, 16/8    (1024)        16.9 -> 17.7
+//   8 x 512 causal, segments 16-512, 32/8     (1024)        20.6 -> 21.6 (two)
 //   1 x 4096 bidirectional, one segment, 32/8 (1024)         147 -> 157  (two)
 //   4 x 8192, mean segment 512, 16/8          (4096)          98 -> 106  (two)
-static int heads_per_block(int G, int mode, int nq, long long tile_heads) {
+static int heads_per_block(int G, int mode, int batch, int nq, long long tile_heads) {
   if (G % 2 || tile_heads <= 256) return 1;
-  if (nq == 1 || tile_heads > 3 * 256) return 2;
+  if (nq == 1 || tile_heads > 4 * 256) return 2;
+  if (tile_heads > 3 * 256) return mode == 0 && batch > 1 && nq >= 8 ? 1 : 2;
   return mode == 0 || tile_heads > 2 * 256 ? 1 : 2;
 }
 
@@ -613,7 +619,7 @@ static FwdArgs fwd_args(const void* q, const void* k, const void* v, int batch, 
   a.Hq = Hq;
   a.Hkv = Hkv;
   a.G = Hq / Hkv;
-  *hpw = heads_per_block(a.G, mode, lay.nq, (long long)batch * lay.nq * Hq);
+  *hpw = heads_per_block(a.G, mode, batch, lay.nq, (long long)batch * lay.nq * Hq);
   a.hchunks = a.G / *hpw;
   a.nq = lay.nq;
   a.nk = lay.nk;

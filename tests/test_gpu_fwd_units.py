@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("hq, hkv", [(16, 8), (32, 8), (16, 2), (12, 4)])
 def test_rows_of_a_large_batch_equal_rows_alone(hq, hkv, mode, t, device):
     """40 rows of t tokens (14 of 641) fill the chip: even groups take two heads per workgroup (more
-    than 768 tiles x heads), a row alone (at most 192) takes one; the group of three takes ring
+    than 1024 tiles x heads), a row alone (at most 192) takes one; the group of three takes ring
     slots of one stage in the batches of 40 (960 and 1440 workgroups), of two alone and at t = 641.
     Out, lse and the gradients of every row are bit-identical, also with the query's norm and
     rotation in the forward: lists of one to eleven stages, odd and even, with segments and padding
